@@ -587,7 +587,7 @@ template <bool kRefine, bool kMask = true>
 __device__ __forceinline__ float split_rsqrt(float dx, float dy, float dz, float e2)
 {
     const float R2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, e2)));
-    const float y = kRefine ? rsqrt_refined(R2) : __builtin_amdgcn_rsqf(R2);
+    const float y = kRefine ? rsqrt_refined(R2) : rsq_f32(R2);
     if constexpr (!kMask) return y;
     return R2 > e2 ? y : 0.0f;
 }
@@ -896,12 +896,12 @@ struct OpSplitTstep {
         float v2 = __builtin_fmaf(uz, uz, __builtin_fmaf(uy, uy, ux * ux));
         const bool mask = R2 > e2;
         // no mask on 1/R: a masked pair's term is zeroed at the end
-        float q1 = __builtin_amdgcn_rsqf(R2);
+        float q1 = rsq_f32(R2);
         float q2 = q1 * q1;
         float phi2 = mt * q1;  // 2 phi: mt is the doubled mass sum
         float w2 = q2 * (phi2 + v2);
         float ga = q2 * __builtin_fmaf(q2, phi2, w2);
-        ga *= r.eta * __builtin_amdgcn_rsqf(w2);
+        ga *= r.eta * rsq_f32(w2);
         w2 = __builtin_fmaf(-ga, rv, w2);
         w2 = mask ? w2 : 0.0f;
         c.sum += w2;
