@@ -233,11 +233,12 @@ struct OpAcc {
         P::q12(T(0), e2u, true, q1, q2);
         return q1;
     }
-    __device__ static bool self_safe(T y0, const Slot& s)
+    __device__ static bool self_safe_m(T y0, T m)
     {
-        const T q3 = ((y0 * y0) * y0) * s.v[0];
+        const T q3 = ((y0 * y0) * y0) * m;
         return __builtin_isfinite(q3);
     }
+    __device__ static bool self_safe(T y0, const Slot& s) { return self_safe_m(y0, s.v[0]); }
     __device__ static void zero(Acc& c) { c.ax = c.ay = c.az = 0; }
     template <bool kU = false, bool kM = true>
     __device__ static __forceinline__ void interact(const IReg& r, const Slot& s, Acc& c,
@@ -398,7 +399,10 @@ struct OpSnapCrackle {
 #pragma unroll
         for (int k = 0; k < 6; ++k) c.s[k] = 0;
     }
-    __device__ static __forceinline__ void interact(const IReg& r, const Slot& s, Acc& c)
+    // The pair's snap and crackle terms t per unit of q3 = 1/R^3 and mass
+    // (interact subtracts m_j q3 t; the j-particle's are the opposite).
+    __device__ static __forceinline__ void pair_terms(const IReg& r, const Slot& s, T (&t)[6],
+                                                      T& q3)
     {
         T dx = r.v[0] - s.v[1];
         T dy = r.v[1] - s.v[2];
@@ -421,7 +425,7 @@ struct OpSnapCrackle {
         T vA = dot3<P>(ux, uy, uz, Ax, Ay, Az);
         T q1, q2;
         P::q12(r2, e2, r2 > T(0), q1, q2);
-        T q3 = q2 * q1;
+        q3 = q2 * q1;
 
         T al = rv * q2;
         T al2 = al * al;
@@ -441,13 +445,16 @@ struct OpSnapCrackle {
         Jx -= mad<P>(ga, dx, mad<P>(al, Ax, be * ux));
         Jy -= mad<P>(ga, dy, mad<P>(al, Ay, be * uy));
         Jz -= mad<P>(ga, dz, mad<P>(al, Az, be * uz));
+        t[0] = Ax; t[1] = Ay; t[2] = Az;
+        t[3] = Jx; t[4] = Jy; t[5] = Jz;
+    }
+    __device__ static __forceinline__ void interact(const IReg& r, const Slot& s, Acc& c)
+    {
+        T t[6], q3;
+        pair_terms(r, s, t, q3);
         q3 *= s.v[0];
-        c.s[0] = nmad<P>(q3, Ax, c.s[0]);
-        c.s[1] = nmad<P>(q3, Ay, c.s[1]);
-        c.s[2] = nmad<P>(q3, Az, c.s[2]);
-        c.s[3] = nmad<P>(q3, Jx, c.s[3]);
-        c.s[4] = nmad<P>(q3, Jy, c.s[4]);
-        c.s[5] = nmad<P>(q3, Jz, c.s[5]);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) c.s[k] = nmad<P>(q3, t[k], c.s[k]);
     }
     __device__ static void flush(Acc&) {}
     __device__ static double get(const Acc& c, int k) { return static_cast<double>(c.s[k]); }
@@ -497,9 +504,9 @@ struct OpTstep {
         for (int f = 0; f < 8; ++f) s.v[f] = a.jp[f][j];
     }
     __device__ static void zero(Acc& c) { c.sum = 0; c.mx = 0; }
-    template <bool kU = false>
-    __device__ static __forceinline__ void interact(const IReg& r, const Slot& s, Acc& c,
-                                                    T e2u = T(0))
+    // The pair frequency w^2, the same for both particles; 0 if masked.
+    template <bool kU>
+    __device__ static __forceinline__ T pair_w2(const IReg& r, const Slot& s, T e2u)
     {
         T dx = r.x - s.v[1];
         T dy = r.y - s.v[2];
@@ -524,7 +531,13 @@ struct OpTstep {
         T ga = q2 * mad<P>(b, phi, w2);
         ga *= P::eta_over_sqrt(r.eta, w2);
         w2 = nmad<P>(ga, rv, w2);
-        w2 = mask ? w2 : T(0);
+        return mask ? w2 : T(0);
+    }
+    template <bool kU = false>
+    __device__ static __forceinline__ void interact(const IReg& r, const Slot& s, Acc& c,
+                                                    T e2u = T(0))
+    {
+        const T w2 = pair_w2<kU>(r, s, e2u);
         c.sum += w2;
         c.mx = fmax_t(w2, c.mx);
     }
@@ -657,11 +670,12 @@ struct OpSplitAccT {
     static constexpr bool kUnmask = true;
     __device__ static bool unmask_allowed(const Args&) { return true; }
     __device__ static float self_y(float e2u) { return split_self_rsqrt<kRefine>(e2u); }
-    __device__ static bool self_safe(float y0, const Slot& s)
+    __device__ static bool self_safe_m(float y0, float m)
     {
-        const float q3 = (y0 * y0) * (y0 * s.v[3]);
+        const float q3 = (y0 * y0) * (y0 * m);
         return __builtin_isfinite(q3);
     }
+    __device__ static bool self_safe(float y0, const Slot& s) { return self_safe_m(y0, s.v[3]); }
     __device__ static void zero(Acc& c)
     {
         c.ax = c.ay = c.az = 0.0f;
@@ -878,9 +892,9 @@ struct OpSplitTstep {
         c.mx = 0.0f;
         c.tsum = 0.0;
     }
-    template <bool kU = false>
-    __device__ static __forceinline__ void interact(const IReg& r, const Slot& s, Acc& c,
-                                                    float e2u = float(0))
+    // As OpTstep::pair_w2.
+    template <bool kU>
+    __device__ static __forceinline__ float pair_w2(const IReg& r, const Slot& s, float e2u)
     {
         float dx = (r.xh - s.v[0]) + (r.xl - s.v[4]);
         float dy = (r.yh - s.v[1]) + (r.yl - s.v[5]);
@@ -903,7 +917,13 @@ struct OpSplitTstep {
         float ga = q2 * __builtin_fmaf(q2, phi2, w2);
         ga *= r.eta * rsq_f32(w2);
         w2 = __builtin_fmaf(-ga, rv, w2);
-        w2 = mask ? w2 : 0.0f;
+        return mask ? w2 : 0.0f;
+    }
+    template <bool kU = false>
+    __device__ static __forceinline__ void interact(const IReg& r, const Slot& s, Acc& c,
+                                                    float e2u = float(0))
+    {
+        const float w2 = pair_w2<kU>(r, s, e2u);
         c.sum += w2;
         c.mx = __builtin_fmaxf(w2, c.mx);
     }

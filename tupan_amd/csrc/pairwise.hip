@@ -8,6 +8,7 @@
 
 #include "ops.h"
 #include "pn.h"
+#include "sym.h"
 #include "tupan_internal.h"
 
 namespace tupan {
@@ -145,6 +146,103 @@ static unsigned coincide_entries(int nj)
     return size;
 }
 
+// The i-set is the j-set: every input array is the same one.
+template <class T>
+static bool same_set(const PairArgs<T>& a)
+{
+    bool same = a.ni == a.nj;
+    for (int f = 0; f < 14; ++f) same = same && a.ip[f] == a.jp[f];
+    return same;
+}
+
+// Whether a call runs the scan, and the workspace bytes it needs (0 if not).
+template <class Op>
+static size_t coincide_bytes(const typename Op::Args& a, const FixedScratch* fixed)
+{
+    if constexpr (HasCoincideScan<Op>::value) {
+        if (!fixed && static_cast<double>(a.ni) * static_cast<double>(a.nj) >= kCoincideMinPairs)
+            return static_cast<size_t>(coincide_entries(a.nj)) * sizeof(int) + 256;
+    }
+    return 0;
+}
+
+// Enqueues the scan in `w` (coincide_bytes) and hands its flag to the call.
+template <class Op>
+static void coincide_scan(typename Op::Args& a, char* w, hipStream_t stream)
+{
+    if constexpr (HasCoincideScan<Op>::value) {
+        const unsigned table_n = coincide_entries(a.nj);
+        int* flag = reinterpret_cast<int*>(w);
+        int* table = flag + 64;
+        const unsigned mask = table_n - 1;
+        hipLaunchKernelGGL(coincide_clear_kernel, dim3((table_n + 255) / 256), dim3(256), 0, stream,
+                           table, table_n, flag);
+        bool same = a.ni == a.nj;
+        for (int f : {1, 2, 3, 5, 6, 7}) same = same && a.ip[f] == a.jp[f];
+        hipLaunchKernelGGL(coincide_insert_kernel<Op>,
+                           dim3(static_cast<unsigned>((a.nj + 255) / 256)), dim3(256), 0, stream, a,
+                           table, mask, flag, same ? 1 : 0);
+        if (!same)
+            hipLaunchKernelGGL(coincide_probe_kernel,
+                               dim3(static_cast<unsigned>((a.ni + 255) / 256)), dim3(256), 0,
+                               stream, a, static_cast<const int*>(table), mask, flag);
+        a.coincide = flag;
+    }
+}
+
+template <class Op, int SH>
+static void launch_sym(const typename Op::Args& a, const SymPlan& p, hipStream_t stream)
+{
+    using S = typename SymOf<Op>::type;
+    hipLaunchKernelGGL((sym_kernel<S, kSymShapeDims[SH][0], kSymShapeDims[SH][1]>),
+                       dim3(static_cast<unsigned>(p.nb * p.nchunk)), dim3(kSymBlock), 0, stream, a,
+                       p.nb);
+}
+
+// A set against itself on the symmetric engine (sym.h); false when the call
+// is not one (ieee64 keeps the reference's sum order), the plan declines it
+// or the scratch does not hold its partial sums: the tile engine takes it.
+template <class Op>
+static bool run_sym(typename Op::Args a, hipStream_t stream, const FixedScratch* fixed, int* rc)
+{
+    if constexpr (kHasSym<Op>) {
+        using S = typename SymOf<Op>::type;
+        if (a.exact || !same_set(a)) return false;
+        const SymPlan p = sym_plan(a.ni, S::kK, sizeof(typename S::T) == 8,
+                                   current_device().cu_count);
+        if (p.shape < 0) return false;
+        const size_t part_bytes = sym_doubles(p, S::kK, a.ni) * sizeof(double);
+        const size_t part_round = (part_bytes + 255) / 256 * 256;
+        const size_t scan_bytes = coincide_bytes<Op>(a, fixed);
+        a.coincide = nullptr;
+        if (fixed) {
+            if (part_bytes > fixed->doubles * sizeof(double)) return false;
+            a.partial = fixed->p;
+        } else {
+            char* w = static_cast<char*>(workspace(part_round + scan_bytes, stream));
+            if (!w) return false;
+            a.partial = reinterpret_cast<double*>(w);
+            if (scan_bytes) coincide_scan<Op>(a, w + part_round, stream);
+        }
+        a.nsplit = p.nchunk;
+        a.jchunk = 0;
+        if (!fixed) timing_begin(stream);
+        switch (p.shape) {
+        case 0: launch_sym<Op, 0>(a, p, stream); break;
+        case 1: launch_sym<Op, 1>(a, p, stream); break;
+        default: launch_sym<Op, 2>(a, p, stream); break;
+        }
+        if (!fixed) timing_end(stream);
+        hipLaunchKernelGGL((sym_reduce_kernel<S>),
+                           dim3(static_cast<unsigned>((a.ni + kWave - 1) / kWave)),
+                           dim3(kSymReduceWaves * kWave), 0, stream, a, p.nb,
+                           kSymBlock * kSymShapeDims[p.shape][0]);
+        *rc = check_launch("pairwise");
+        return true;
+    }
+    return false;
+}
+
 template <class Op, int BLOCK, int WPT, int TILE, int UNROLL>
 static int run_pairwise(typename Op::Args a, hipStream_t stream, int wg_per_cu,
                         const FixedScratch* fixed)
@@ -185,15 +283,11 @@ static int run_pairwise(typename Op::Args a, hipStream_t stream, int wg_per_cu,
     a.partial = nullptr;
     a.coincide = nullptr;
     // the coincidence table and flag follow the partials in the workspace
-    bool scan = false;
-    if constexpr (HasCoincideScan<Op>::value)
-        scan = !fixed && static_cast<double>(a.ni) * static_cast<double>(a.nj) >= kCoincideMinPairs;
+    const size_t scan_bytes = coincide_bytes<Op>(a, fixed);
     const size_t part_bytes =
         L.nsplit > 1 ? static_cast<size_t>(L.nsplit) * Op::kNacc * a.ni * sizeof(double) : 0;
     const size_t part_round = (part_bytes + 255) / 256 * 256;
-    const unsigned table_n = scan ? coincide_entries(a.nj) : 0u;
-    const size_t scan_bytes = scan ? static_cast<size_t>(table_n) * sizeof(int) + 256 : 0;
-    if (L.nsplit > 1 || scan) {
+    if (L.nsplit > 1 || scan_bytes) {
         if (fixed) {
             if (part_bytes > fixed->doubles * sizeof(double))
                 return set_error(TUPAN_ERR_ARG, "j-split partials exceed the fixed scratch");
@@ -202,26 +296,7 @@ static int run_pairwise(typename Op::Args a, hipStream_t stream, int wg_per_cu,
             char* w = static_cast<char*>(workspace(part_round + scan_bytes, stream));
             if (!w) return set_error(TUPAN_ERR_ALLOC, "workspace allocation failed");
             if (L.nsplit > 1) a.partial = reinterpret_cast<double*>(w);
-            if constexpr (HasCoincideScan<Op>::value) {
-                if (scan) {
-                    int* flag = reinterpret_cast<int*>(w + part_round);
-                    int* table = flag + 64;
-                    const unsigned mask = table_n - 1;
-                    hipLaunchKernelGGL(coincide_clear_kernel, dim3((table_n + 255) / 256),
-                                       dim3(256), 0, stream, table, table_n, flag);
-                    bool same = a.ni == a.nj;
-                    for (int f : {1, 2, 3, 5, 6, 7}) same = same && a.ip[f] == a.jp[f];
-                    hipLaunchKernelGGL(coincide_insert_kernel<Op>,
-                                       dim3(static_cast<unsigned>((a.nj + 255) / 256)), dim3(256),
-                                       0, stream, a, table, mask, flag, same ? 1 : 0);
-                    if (!same)
-                        hipLaunchKernelGGL(coincide_probe_kernel,
-                                           dim3(static_cast<unsigned>((a.ni + 255) / 256)),
-                                           dim3(256), 0, stream, a,
-                                           static_cast<const int*>(table), mask, flag);
-                    a.coincide = flag;
-                }
-            }
+            if (scan_bytes) coincide_scan<Op>(a, w + part_round, stream);
         }
     }
     const unsigned grid = static_cast<unsigned>(L.nblock_i) * static_cast<unsigned>(L.nsplit);
@@ -311,6 +386,8 @@ template <class Op>
 static int launch_tuned(const Launcher<Op> (&table)[kShapes], int kernel, int slot,
                         typename Op::Args& a, hipStream_t s, const FixedScratch* fixed)
 {
+    int rc = TUPAN_OK;
+    if (run_sym<Op>(a, s, fixed, &rc)) return rc;
     const TuneEntry& t = g_tune[kernel][slot][size_bucket(a.ni, a.nj)];
     const int shape = (t.shape >= 0 && t.shape < kShapes) ? t.shape : 0;
     return table[shape](a, s, t.wg_per_cu, fixed);

@@ -28,7 +28,7 @@
 // Compiled with -ffp-contract=off.
 #include "block_step.h"
 #include "kepler.h"
-#include "ops.h"
+#include "sym.h"
 #include "tupan_internal.h"
 
 namespace tupan {
@@ -517,6 +517,7 @@ constexpr int kLvlIter = 1024;       // scheduler transitions per slot
 constexpr int kLvlVisits = 1 << 20;  // level visits per step
 constexpr int kPartPer = 1024;       // particles per partition block (256 x 4)
 constexpr int kCandSmall = kNumShapes;  // candidate id of the small-set kernel
+constexpr int kCandSym = kNumShapes + 1;  // of the symmetric engine's first shape
 
 enum { LK_NONE = 0, LK_PAIR = 1, LK_PART = 2, LK_ELEM = 3, LK_SUBTREE = 4, LK_FEW = 5 };
 enum { MT_TSTEP, MT_ACC, MT_PART, MT_DRIFT, MT_KICK, MT_FEW, MT_PUSH };
@@ -544,7 +545,7 @@ struct LvlCtl {
     int sp, qh, qt;
     int done, status, visits, ops;  // ops: slots that did work this step
     // this slot's operation
-    int kind, op, cand, grid, comb, comb_grid, elem;
+    int kind, op, cand, grid, comb, comb_grid, elem, sym_nb;
     int lo, n, ns;
     double h, tau;
     PairArgs<double> pa;
@@ -625,6 +626,21 @@ __device__ void lvl_plan(LvlCtl* c, int op, int ilo, int ni, int jlo, int nj)
         constexpr int ipb = kSmallBlock / kSmallGroups;
         c->grid = (ni + ipb - 1) / ipb;
         return;
+    }
+    if (ilo == jlo && ni == nj) {
+        const bool fp64 = (op == 0 ? c->tstep_mode : c->acc_mode) != TUPAN_MODE_SPLIT32;
+        const SymPlan sp = sym_plan(ni, op == 0 ? 2 : 3, fp64, c->cu_count);
+        if (sp.shape >= 0) {
+            a.nsplit = sp.nchunk;
+            a.jchunk = 0;
+            a.partial = c->partial;
+            c->cand = kCandSym + sp.shape;
+            c->grid = sp.nb * sp.nchunk;
+            c->sym_nb = sp.nb;
+            c->comb = 3;
+            c->comb_grid = (ni + kWave - 1) / kWave;
+            return;
+        }
     }
     const int b = lvl_bucket(ni, nj);
     const int shape = c->tshape[op][b];
@@ -832,6 +848,27 @@ __global__ __launch_bounds__(kSmallBlock) void lvl_small_kernel(const LvlCtl* c,
     const int bid = static_cast<int>(blockIdx.x);
     if (bid >= c->grid) return;
     pair_small_body<Op, kSmallBlock, kSmallGroups, small_tile<Op>()>(c->pa, bid);
+}
+
+template <class Op, int S>
+__global__ __launch_bounds__(kSymBlock) void lvl_sym_kernel(const LvlCtl* c, int op)
+{
+    if (c->kind != LK_PAIR || c->op != op || c->cand != kCandSym + S) return;
+    const int bid = static_cast<int>(blockIdx.x);
+    if (bid >= c->grid) return;
+    sym_body<typename SymOf<Op>::type, kSymShapeDims[S][0], kSymShapeDims[S][1]>(c->pa, bid,
+                                                                                 c->sym_nb);
+}
+
+template <class Op>
+__global__ __launch_bounds__(kSymReduceWaves* kWave) void lvl_sym_reduce_kernel(const LvlCtl* c,
+                                                                                int op)
+{
+    if (c->kind != LK_PAIR || c->op != op || c->comb != 3) return;
+    const int bid = static_cast<int>(blockIdx.x);
+    if (bid >= c->comb_grid) return;
+    sym_reduce_body<typename SymOf<Op>::type>(
+        c->pa, bid, c->sym_nb, kSymBlock * kSymShapeDims[c->cand - kCandSym][0]);
 }
 
 template <class Op>
@@ -1043,6 +1080,7 @@ struct LevelsPlan {
     int tstep_mode = 0, acc_mode = 0;
     int shapes[2][kNumShapes] = {};   // shapes the tuning table uses, per op
     int grid_max[2][kNumShapes] = {};
+    int sym_grid[2][kNumSymShapes] = {};  // largest grids of the symmetric engine, 0: unused
 };
 
 int sia_levels_create(int n, void* const* arrays, int narrays, const int* roles, int acc_mode,
@@ -1125,6 +1163,26 @@ int sia_levels_create(int n, void* const* arrays, int narrays, const int* roles,
             if (need > part_doubles) part_doubles = need;
         }
     }
+    // the symmetric engine's largest grid per shape and its partial sums over
+    // every set size: a plan's counts depend on the size through its block
+    // count, so the multiples of the smallest block and n cover them
+    for (int op = 0; op < 2; ++op) {
+        const int nacc = op == 0 ? 2 : 3;
+        const bool fp64 = (op == 0 ? tstep_mode : acc_mode) != TUPAN_MODE_SPLIT32;
+        for (long long q = kSymBlock;; q += kSymBlock) {
+            const int m = static_cast<int>(q < n ? q : n);
+            const int shape = sym_shape(m, fp64);
+            if (shape >= 0) {
+                const SymPlan sp = sym_plan(m, nacc, fp64, h.cu_count);
+                const int grid = sp.nb * sp.nchunk;
+                if (grid > p->sym_grid[op][shape]) p->sym_grid[op][shape] = grid;
+                size_t need = sym_doubles(sp, nacc, m);
+                if (need > kSymMaxBytes / sizeof(double)) need = kSymMaxBytes / sizeof(double);
+                if (need > part_doubles) part_doubles = need;
+            }
+            if (m == n) break;
+        }
+    }
     const size_t nb = (static_cast<size_t>(n) + kPartPer - 1) / kPartPer;
     int rc = check_hip(hipMalloc(&p->ctl, sizeof(LvlCtl)), "levels control");
     if (rc == TUPAN_OK)
@@ -1170,8 +1228,8 @@ namespace {
 template <class Op>
 int lvl_enqueue_pair_workers(const LevelsPlan* p, int op, hipStream_t s)
 {
-    // one launch per shape the tuning table uses, the small-set kernel and
-    // the two combines
+    // one launch per shape the tuning table uses, the small-set kernel, the
+    // two combines, the symmetric engine's shapes and its reduction
 #define TUPAN_LVL_SHAPE(S)                                                                   \
     if (p->shapes[op][S])                                                                    \
         hipLaunchKernelGGL((lvl_pair_kernel<Op, S>), dim3(p->grid_max[op][S]),               \
@@ -1192,6 +1250,17 @@ int lvl_enqueue_pair_workers(const LevelsPlan* p, int op, hipStream_t s)
                        dim3(256), 0, s, p->ctl, op, 1);
     hipLaunchKernelGGL((lvl_combine_kernel<Op>), dim3((p->N + 255) / 256), dim3(256), 0, s,
                        p->ctl, op, 0);
+#define TUPAN_LVL_SYM(S)                                                                     \
+    if (p->sym_grid[op][S])                                                                  \
+        hipLaunchKernelGGL((lvl_sym_kernel<Op, S>), dim3(p->sym_grid[op][S]),                \
+                           dim3(kSymBlock), 0, s, p->ctl, op);
+    TUPAN_LVL_SYM(0)
+    TUPAN_LVL_SYM(1)
+    TUPAN_LVL_SYM(2)
+#undef TUPAN_LVL_SYM
+    if (p->sym_grid[op][0] || p->sym_grid[op][1] || p->sym_grid[op][2])
+        hipLaunchKernelGGL((lvl_sym_reduce_kernel<Op>), dim3((p->N + kWave - 1) / kWave),
+                           dim3(kSymReduceWaves * kWave), 0, s, p->ctl, op);
     return check_launch("levels pair workers");
 }
 

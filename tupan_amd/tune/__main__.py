@@ -69,7 +69,10 @@ def tune_pairwise(quick, names):
     # PNAcc at the reference's own test values (order 7, c = 128)
     extensions.clight.pn_order, extensions.clight.clight = 7, 128.0
     for b, n in enumerate(sizes):
+        # the table serves calls between two sets (a set against itself
+        # above ~2000 particles takes the symmetric engine's own plan)
         ps = cluster(n)
+        other = ps.copy()
         for name, (kid, modes) in KERNELS.items():
             if name not in names:
                 continue
@@ -87,7 +90,7 @@ def tune_pairwise(quick, names):
                         _native.check(lib.tupan_tune_set(kid, SLOT[mode], b,
                                                          shape, wg),
                                       "tupan_tune_set")
-                        t = time_call(lambda: ext.calc(ps, ps, *args), 3)
+                        t = time_call(lambda: ext.calc(ps, other, *args), 3)
                         results.append((t, shape, wg))
                 results.sort()
                 t, shape, wg = results[0]
