@@ -547,8 +547,19 @@ __host__ __device__ inline int min_jchunk(int nj, int tile, bool exact)
     return nj > tile ? 32 : tile;
 }
 
+// At most max_split splits; 64 by default, and as many as there are whole
+// tiles where few i-blocks meet many j (a block-step level's slow <-> fast
+// force): 64 x 5 workgroups for 2501 x 60000 left the 256 CUs with one or
+// two each (split Acc 114 us, 97 with 111 x 5; FP64 Acc 30 x 262144 382 -> 115 us).
+__host__ __device__ inline int split_limit(int nj, int tile)
+{
+    const int t = nj / tile;
+    return t > 64 ? t : 64;
+}
+
 __host__ __device__ inline Launch plan_launch(int ni, int nj, int block, int wpt, int tile,
-                                              int target_wg, int max_split, int min_chunk)
+                                              int target_wg, int max_split, int min_chunk,
+                                              int cu = 0)
 {
     Launch L;
     const int per_block = block * wpt;
@@ -563,6 +574,25 @@ __host__ __device__ inline Launch plan_launch(int ni, int nj, int block, int wpt
     int chunk = (nj + ns - 1) / ns;
     chunk = ((chunk + min_chunk - 1) / min_chunk) * min_chunk;
     if (chunk < min_chunk) chunk = min_chunk;
+    // a few workgroups per CU: of the chunk lengths down to half of that the
+    // one whose busiest CU has the least to do (a workgroup's fixed cost
+    // counted as kSplitFixed j)
+    constexpr int kSplitFixed = 64;
+    if (cu > 0 && ns > 1 && L.nblock_i * ns < 8 * cu) {
+        long long best = -1;
+        int pick = chunk;
+        for (int c = chunk; c >= min_chunk && 2 * c >= chunk; c -= min_chunk) {
+            const int n = (nj + c - 1) / c;
+            if (n > max_split) break;
+            const long long cost =
+                static_cast<long long>((L.nblock_i * n + cu - 1) / cu) * (c + kSplitFixed);
+            if (best < 0 || cost < best) {
+                best = cost;
+                pick = c;
+            }
+        }
+        chunk = pick;
+    }
     L.jchunk = chunk;
     L.nsplit = nj > 0 ? (nj + chunk - 1) / chunk : 1;
     return L;

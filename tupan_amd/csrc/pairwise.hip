@@ -270,14 +270,15 @@ static int run_pairwise(typename Op::Args a, hipStream_t stream, int wg_per_cu,
     // below 256 particles, so any set of at most 256 is one split (the
     // reference's summation order) whatever shape is tuned.
     const int min_chunk = min_jchunk(a.nj, TILE, a.exact != 0);
-    // at most 64 j-splits; with lent scratch, at most as many as it holds
-    int max_split = 64;
+    // with lent scratch, at most as many j-splits as it holds
+    int max_split = split_limit(a.nj, TILE);
     if (fixed) {
         const size_t per_split = static_cast<size_t>(Op::kNacc) * static_cast<size_t>(a.ni);
         const size_t fit = fixed->doubles / per_split;
         if (fit < static_cast<size_t>(max_split)) max_split = fit > 1 ? static_cast<int>(fit) : 1;
     }
-    Launch L = plan_launch(a.ni, a.nj, BLOCK, WPT, TILE, target, max_split, min_chunk);
+    Launch L = plan_launch(a.ni, a.nj, BLOCK, WPT, TILE, target, max_split, min_chunk,
+                           a.exact ? 0 : dev.cu_count);
     a.nsplit = L.nsplit;
     a.jchunk = L.jchunk;
     a.partial = nullptr;

@@ -649,7 +649,8 @@ __device__ void lvl_plan(LvlCtl* c, int op, int ilo, int ni, int jlo, int nj)
               TILE = kLightShapeDims[shape][2];
     const int target = (wg > 0 ? wg : 4) * c->cu_count;
     const int min_chunk = min_jchunk(nj, TILE, false);
-    const Launch L = plan_launch(ni, nj, BLOCK, WPT, TILE, target, 64, min_chunk);
+    const Launch L = plan_launch(ni, nj, BLOCK, WPT, TILE, target, split_limit(nj, TILE), min_chunk,
+                                 c->cu_count);
     a.nsplit = L.nsplit;
     a.jchunk = L.jchunk;
     c->cand = shape;
@@ -1155,11 +1156,11 @@ int sia_levels_create(int n, void* const* arrays, int narrays, const int* roles,
             const int ipb = kLightShapeDims[s][0] * kLightShapeDims[s][1];
             const long long target = static_cast<long long>(wg_max[op][s]) * h.cu_count;
             const long long nblk = (n + ipb - 1) / ipb;
-            p->grid_max[op][s] = static_cast<int>(target + nblk + 1);
-            // nsplit * ni <= min(64 ni, (target / nblock_i + 1) * nblock_i * ipb)
-            const size_t a = static_cast<size_t>(64) * n;
-            const size_t b = static_cast<size_t>(target + nblk) * ipb;
-            const size_t need = nacc * (a < b ? a : b);
+            // plan_launch: nblock_i * nsplit is at most target + nblock_i, or
+            // twice a count below 8 per CU, plus nblock_i
+            const long long few = 16ll * h.cu_count;
+            p->grid_max[op][s] = static_cast<int>((target > few ? target : few) + nblk + 1);
+            const size_t need = nacc * static_cast<size_t>(p->grid_max[op][s]) * ipb;
             if (need > part_doubles) part_doubles = need;
         }
     }
