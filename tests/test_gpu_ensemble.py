@@ -170,3 +170,41 @@ def test_ensemble_graph_replay_equals_eager():
     assert a.nsteps == b.nsteps == 16 and a.time == b.time
     for k in keys:
         assert torch.equal(getattr(ps3, k), getattr(ps4, k)), k
+
+
+def test_every_small_size_counts_each_ordered_pair():
+    """Each unordered pair is drifted once and counted for both particles:
+    sizes 1 to 12 (odd, even, alone) and around the lane groups, increments
+    against the oracle and solves + leapfrogs = n (n - 1) per system; a
+    massless particle's own term stays NaN, as in the reference's loop."""
+    from oracle import Oracle
+    from tupan_amd.lib.ensemble import Ensemble
+    from tupan_amd.particles import ParticleSystem
+    sizes = list(range(1, 13)) + [31, 32, 33, 63, 64]
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    n = int(off[-1])
+    rng = np.random.default_rng(21)
+    d = {k: rng.normal(0, 1, n) for k in ("rx", "ry", "rz")}
+    d.update({k: rng.normal(0, 0.6, n) for k in ("vx", "vy", "vz")})
+    d["mass"] = rng.random(n) * 0.1 + 0.01
+    d["eps2"] = np.zeros(n)
+    ps = ParticleSystem.from_numpy(d, device="cuda:0")
+    ens = Ensemble(off)
+    ens.counters = torch.zeros(4, dtype=torch.int64, device="cuda:0")
+    orc = Oracle("float64")
+    got = [t.cpu().numpy().copy() for t in ens.sakura(ps, 1.0 / 64, -1)]
+    for s in range(len(sizes)):
+        a, b = off[s], off[s + 1]
+        sub = {k: v[a:b] for k, v in d.items()}
+        ref = orc.sakura(sub, sub, 1.0 / 64, -1)
+        if sizes[s] == 1:
+            assert all(np.all(g[a:b] == 0) for g in got)
+            continue
+        assert vec_rel_err([g[a:b] for g in got[:3]], ref[:3]) <= 1e-9
+        assert vec_rel_err([g[a:b] for g in got[3:]], ref[3:]) <= 1e-9
+    c = ens.counters.cpu().tolist()
+    assert c[2] == 0 and c[0] + c[3] == sum(k * (k - 1) for k in sizes)
+    ps.mass[1] = 0.0  # one of the two-particle system
+    got = ens.sakura(ps, 1.0 / 64, -1, check=False)
+    assert all(bool(torch.isnan(g[1])) for g in got)
+    assert all(bool(torch.isfinite(g[2:]).all()) for g in got)

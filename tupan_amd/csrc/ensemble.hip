@@ -7,23 +7,24 @@
 // systems are sorted by size and each size bucket gets L lanes per system
 // (L in {8, 16, 32, 64}, at least the system size), so a wave holds 64/L
 // systems of similar size.  Lane l of a wave serves particle l % L of
-// system l / L and loops over that system's j particles.  The lanes of a
-// wave step through their j loops together, so each step lasts as long as
-// the slowest Kepler solve among the wave's pairs at that step; grouping
-// systems of similar size keeps the lanes' loop lengths close.  Every lane
+// system l / L and meets the others in rounds.  The lanes of a
+// wave step through their rounds together, so each lasts as long as
+// the slowest Kepler solve among the wave's pairs in it; grouping
+// systems of similar size keeps the lanes' round counts close.  Every lane
 // stays in the wave to the end (inactive lanes compute nothing), so the
 // wave reductions of the work counters see all 64 lanes.
 //
 // With a Kepler-guess network set on the plan (ensemble_plan_set_guess)
-// the launch takes the learned form: each j step first evaluates the
+// the launch takes the learned form: each round first evaluates the
 // network on the wave's 64 pairs (mlp_wave.h, the same inference as the
 // Sakura near pass) and every pair's first solve starts from its guess.
-// The network needs all 64 lanes, so each lane runs the wave's longest j
-// loop, idle past its own range.
+// The network needs all 64 lanes, so each lane runs the wave's longest
+// share of rounds, idle past its own.
 //
 // The Sakura drift runs each plan wave as one workgroup of kEnsParts waves:
-// wave p takes the p-th of kEnsParts consecutive j ranges of the same lanes,
-// and the partial sums are added in part order (((d0 + d1) + d2) + d3), so a
+// wave p takes the p-th of kEnsParts consecutive shares of the same lanes'
+// rounds (ensemble_sakura_body), and the partial sums are added in part order
+// (((d0 + d1) + d2) + d3), so a
 // launch has kEnsParts times as many, shorter waves to hide the solver's
 // latency with (4 570 -> 12 416 waves for 4096 systems of U{3..64}).
 //
@@ -112,11 +113,13 @@ struct EnsI {
     double m, x, y, z, e2, vx, vy, vz;
 };
 
-// One pair drift of particle i against j (sakura_kernel_common.h:194-243),
-// its increments weighted by m_j / (m_i + m_j) added to d.
+// One pair drift of particle i against j (sakura_kernel_common.h:194-243):
+// its increments weighted by m_j / (m_i + m_j) added to i's sums d, and
+// weighted by -m_i / (m_i + m_j) given as j's in o (the relative orbit of j
+// about i is the mirror image: every increment changes sign and nothing else).
 __device__ __forceinline__ void ens_pair_drift(const EnsArgs& a, const EnsI& I, int j,
                                                const kep::Guess* guess, kep::Counters& cnt,
-                                               double d[6])
+                                               double d[6], double o[6])
 {
     const double jm = a.p[0][j];
     const double p0[3] = {I.x - a.p[1][j], I.y - a.p[2][j], I.z - a.p[3][j]};
@@ -126,13 +129,14 @@ __device__ __forceinline__ void ens_pair_drift(const EnsArgs& a, const EnsI& I, 
     double p[3] = {p0[0], p0[1], p0[2]};
     double v[3] = {v0[0], v0[1], v0[2]};
     kep::drift_twobody(a.dt, a.flag, m, e2, p, v, cnt, guess);
-    const double mu = jm / m;
-    d[0] += mu * (p[0] - p0[0]);
-    d[1] += mu * (p[1] - p0[1]);
-    d[2] += mu * (p[2] - p0[2]);
-    d[3] += mu * (v[0] - v0[0]);
-    d[4] += mu * (v[1] - v0[1]);
-    d[5] += mu * (v[2] - v0[2]);
+    const double mu = jm / m, nu = -(I.m / m);
+    const double c[6] = {p[0] - p0[0], p[1] - p0[1], p[2] - p0[2],
+                         v[0] - v0[0], v[1] - v0[1], v[2] - v0[2]};
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        d[k] += mu * c[k];
+        o[k] = nu * c[k];
+    }
 }
 
 // The network inputs of pair (i, j): the first twobody stage's features
@@ -153,6 +157,14 @@ __device__ __forceinline__ void ens_guess_inputs(const EnsArgs& a, const EnsI& I
     prepare_features(f.tau, f.sigma, f.kappa, f.eps, net->mean, net->inv_std, xs);
 }
 
+// Each unordered pair of a system is drifted once: in round q (q = 0 .. n/2)
+// particle l meets particle l + q (mod n) and hands it the mirrored
+// increments through a lane exchange, so a system of n takes n/2 + 1 rounds
+// instead of n.  Round 0 is the particle with itself (zero, or NaN for a
+// massless or non-finite particle, as in the reference's loop over every j);
+// in the last round of an even n the first half of the lanes covers every
+// pair.  A round's solves bound its time, and their number is what the split
+// halves: 4096 systems of U{3..64}, one flag -1 stage: 0.472 -> 0.283 ms.
 template <bool kLearned>
 __device__ __forceinline__ void ensemble_sakura_body(const EnsArgs& a)
 {
@@ -163,56 +175,88 @@ __device__ __forceinline__ void ensemble_sakura_body(const EnsArgs& a)
     const int part = static_cast<int>(threadIdx.x) / kWave;
     const int lane = static_cast<int>(threadIdx.x) % kWave;
     const EnsLane L = ens_lane(a, wave, lane);
+    // a pair counts for both particles (doubled below)
     kep::Counters cnt;
     double d[6] = {0, 0, 0, 0, 0, 0};
-    int ja = 0, jb = 0;
+    int n = 0, il = 0, qa = 0, qb = 0;
     EnsI I{};
     if (L.active) {
         const int i = L.i;
-        const int nj = L.j1 - L.j0;
-        ja = L.j0 + (nj * part) / kEnsParts;
-        jb = L.j0 + (nj * (part + 1)) / kEnsParts;
+        n = L.j1 - L.j0;
+        il = i - L.j0;
+        const int rounds = n / 2 + 1;
+        qa = (rounds * part) / kEnsParts;
+        qb = (rounds * (part + 1)) / kEnsParts;
         I = EnsI{a.p[0][i], a.p[1][i], a.p[2][i], a.p[3][i],
                  a.p[4][i], a.p[5][i], a.p[6][i], a.p[7][i]};
     }
-    if constexpr (kLearned) {
-        __shared__ __align__(16) NetPacked lnet;
-        mlp_stage(a.net, &lnet);
-        int steps = jb - ja;
+    // the wave's longest share of rounds: every lane takes part in the
+    // exchanges
+    int steps = qb - qa;
 #pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1)
-            steps = max(steps, __shfl_xor(steps, off, kWave));
-        for (int k = 0; k < steps; ++k) {
+    for (int off = kWave / 2; off > 0; off >>= 1)
+        steps = max(steps, __shfl_xor(steps, off, kWave));
+    [[maybe_unused]] NetPacked* lnet = nullptr;
+    if constexpr (kLearned) {
+        __shared__ __align__(16) NetPacked lds_net;
+        lnet = &lds_net;
+        mlp_stage(a.net, lnet);
+    }
+    for (int k = 0; k < steps; ++k) {
+        const int q = qa + k;
+        const bool in = q < qb;
+        const bool has = in && !(2 * q == n && il >= q);
+        int jl = il + q;
+        if (jl >= n) jl -= n;
+        double o[6] = {0, 0, 0, 0, 0, 0};
+        if constexpr (kLearned) {
             // the weights are read from LDS as the network uses them, not
-            // hoisted out of the j loop and kept live across the solves
+            // hoisted out of the loop and kept live across the solves
             __asm__ volatile("" ::: "memory");
-            const bool has = ja + k < jb;
             float xs[4] = {0.f, 0.f, 0.f, 0.f};
-            if (has) ens_guess_inputs(a, I, ja + k, &lnet, xs);
+            if (has) ens_guess_inputs(a, I, L.j0 + jl, lnet, xs);
             // lanes l and l + 32 supply the B operands of items l mod 32
             // and 32 + l mod 32
             float x[2][4];
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    x[c][q] = __shfl(xs[q], 32 * c + (lane & 31), kWave);
+                for (int t = 0; t < 4; ++t)
+                    x[c][t] = __shfl(xs[t], 32 * c + (lane & 31), kWave);
             }
             float y[2];
-            mlp_wave_eval(&lnet, x, lane, y);
-            const float dl = mlp_delta(&lnet, lane < 32 ? y[0] : y[1]);
+            mlp_wave_eval(lnet, x, lane, y);
+            const float dl = mlp_delta(lnet, lane < 32 ? y[0] : y[1]);
             if (has) {
                 kep::Guess gs;
                 gs.use = dl == dl && dl > -0.9f && dl < 8.0f;
                 gs.delta = static_cast<double>(dl);
-                ens_pair_drift(a, I, ja + k, &gs, cnt, d);
+                ens_pair_drift(a, I, L.j0 + jl, &gs, cnt, d, o);
             }
+        } else {
+            if (has) ens_pair_drift(a, I, L.j0 + jl, nullptr, cnt, d, o);
         }
+        // the increments of the particle that met this one: lane - q of the
+        // system (round 0 is the particle itself)
+        int sl = il - q;
+        if (sl < 0) sl += n;
+        const int src = in ? lane - il + sl : lane;
+        const bool take = in && q > 0;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            const double t = __shfl(o[c], src, kWave);
+            if (take) d[c] += t;
+        }
+    }
+    cnt.solves *= 2;
+    cnt.iters *= 2;
+    cnt.retries *= 2;
+    cnt.leapfrog *= 2;
+    cnt.fallbacks *= 2;
+    if constexpr (kLearned) {
         const unsigned int fb = ens_wave_sum(L.active ? cnt.fallbacks : 0u);
         if (lane == 0 && fb && a.fallbacks)
             atomicAdd(a.fallbacks, static_cast<unsigned long long>(fb));
-    } else {
-        for (int j = ja; j < jb; ++j) ens_pair_drift(a, I, j, nullptr, cnt, d);
     }
     if (part > 0) {
 #pragma unroll
