@@ -482,6 +482,25 @@ int tupan_sia_subtree(int n, void *const *arrays, int narrays, const int *roles,
                       double *t_curr, unsigned long long *pairs, int *status,
                       void *stream);
 
+/* Level operations of the host-driven hierarchical SIA steps
+ * (tupan/integrator/sia.py:24-171, 1089-1123), one call for what the
+ * reference does array by array.
+ *
+ * tupan_sia_split: stable in-place partition of every array (8-byte elements,
+ * 1 to 32 of them, n >= 1 values each) to [slow | fast], slow where
+ * |tstep[i]| > threshold; tstep may be one of the arrays.  Waits for the
+ * stream and writes out[0] = slow particles, out[1] = *status (a device
+ * word; 0 if status is null) on the host.
+ *
+ * tupan_sia_update: kind 0, arrays {x0, x1, x2, v0, v1, v2}: x += v h;
+ * kind 1, arrays {tstep, time, nstep (int64)}: tstep = h, time += h,
+ * nstep += 1. */
+int tupan_sia_split(size_t n, void *const *arrays, int narrays,
+                    const double *tstep, double threshold, const int *status,
+                    int *out, void *stream);
+int tupan_sia_update(int kind, size_t n, void *const *arrays, double h,
+                     void *stream);
+
 /* Device-driven shared-step SIA steps: the 's' (fixed step) and 'a'
  * (adaptive block step) variants of the SIA methods
  * (tupan/integrator/sia.py:1089-1123 with the block step of

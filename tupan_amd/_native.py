@@ -143,6 +143,12 @@ def _declare(lib):
                                        ctypes.c_double, ctypes.c_double,
                                        ctypes.c_int, _P, _P, ctypes.c_int, _P,
                                        _P, _P, _P, _P, _P])
+    lib.tupan_sia_split.restype = ctypes.c_int
+    lib.tupan_sia_split.argtypes = [_S, _PP, ctypes.c_int, _P, ctypes.c_double,
+                                    _P, IP, _P]
+    lib.tupan_sia_update.restype = ctypes.c_int
+    lib.tupan_sia_update.argtypes = [ctypes.c_int, _S, _PP, ctypes.c_double,
+                                     _P]
     lib.tupan_mlp_sizes.restype = ctypes.c_int
     lib.tupan_mlp_sizes.argtypes = [ctypes.POINTER(ctypes.c_int)] * 3
     lib.tupan_mlp_grad.restype = ctypes.c_int
@@ -259,6 +265,7 @@ DEVICE_ABI = ("tupan_last_error", "tupan_version", "tupan_device_info",
               "tupan_pnacc", "tupan_pnacc_f32", "tupan_host_pnacc_f32",
               "tupan_hermite_step", "tupan_sakura_graph",
               "tupan_sakura_step", "tupan_sia_step",
+              "tupan_sia_split", "tupan_sia_update",
               "tupan_sia_levels_create", "tupan_sia_levels_destroy",
               "tupan_sia_levels_set", "tupan_sia_levels_enqueue",
               "tupan_sia_levels_state")

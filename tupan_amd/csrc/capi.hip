@@ -873,6 +873,17 @@ int tupan_sia_subtree(int n, void* const* arrays, int narrays, const int* roles,
                             status, stream);
 }
 
+int tupan_sia_split(size_t n, void* const* arrays, int narrays, const double* tstep,
+                    double threshold, const int* status, int* out, void* stream)
+{
+    return sia_split_call(n, arrays, narrays, tstep, threshold, status, out, stream);
+}
+
+int tupan_sia_update(int kind, size_t n, void* const* arrays, double h, void* stream)
+{
+    return sia_update_call(kind, n, arrays, h, stream);
+}
+
 int tupan_kepler_pairs(size_t npairs, const int* idx, const double* m, double* rx, double* ry,
                        double* rz, const double* e2, double* vx, double* vy, double* vz,
                        double dt, int* status, void* stream)

@@ -482,6 +482,215 @@ int sia_step_call(int adaptive, int acc_mode, int tstep_mode, size_t n, void* co
 }  // namespace tupan
 
 // ===========================================================================
+// Level operations of the host-driven hierarchical steps: the stable
+// [slow | fast] partition of every array of a level, and its elementwise
+// updates.  A level visit of a few hundred to a few thousand particles is
+// all launch overhead: as separate array operations the partition was some
+// forty launches (an index list of each part, a gather and a copy per
+// array) and two waits, 360 us, and a drift or kick six launches, 28 us.
+// Here the partition is three launches and one wait, an update one launch.
+// The values are the separate operations', bit for bit.
+// ===========================================================================
+namespace tupan {
+
+namespace {
+
+constexpr int kSplitArrays = 32;
+constexpr int kSplitPer = 1024;  // particles per partition block (256 x 4)
+
+struct SplitArgs {
+    unsigned long long* arr[kSplitArrays];
+    unsigned long long* tmp;  // narr x n
+    const double* tstep;
+    const int* status;  // device status word to hand to the host, or null
+    int* blk;           // slow particles per block
+    int* out;           // slow particles, status
+    double threshold;
+    int n, narr;
+};
+
+__device__ __forceinline__ bool split_slow(const SplitArgs& a, int i)
+{
+    return i < a.n && fabs(a.tstep[i]) > a.threshold;
+}
+
+// Sum over the 256 threads of the block.
+__device__ __forceinline__ int split_block_sum(int v, int* lds)
+{
+    const int t = static_cast<int>(threadIdx.x);
+    lds[t] = v;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if (t < w) lds[t] += lds[t + w];
+        __syncthreads();
+    }
+    const int r = lds[0];
+    __syncthreads();
+    return r;
+}
+
+__global__ __launch_bounds__(256) void sia_split_count_kernel(SplitArgs a)
+{
+    __shared__ int lds[256];
+    const int base = static_cast<int>(blockIdx.x) * kSplitPer + static_cast<int>(threadIdx.x) * 4;
+    int cnt = 0;
+    for (int u = 0; u < 4; ++u) cnt += split_slow(a, base + u) ? 1 : 0;
+    const int sum = split_block_sum(cnt, lds);
+    if (threadIdx.x == 0) a.blk[blockIdx.x] = sum;
+}
+
+__global__ __launch_bounds__(256) void sia_split_scatter_kernel(SplitArgs a)
+{
+    __shared__ int lds[256];
+    const int t = static_cast<int>(threadIdx.x);
+    const int b = static_cast<int>(blockIdx.x);
+    int before = 0, all = 0;
+    for (int k = t; k < static_cast<int>(gridDim.x); k += 256) {
+        all += a.blk[k];
+        if (k < b) before += a.blk[k];
+    }
+    before = split_block_sum(before, lds);
+    const int ns = split_block_sum(all, lds);
+    if (b == 0 && t == 0) {
+        a.out[0] = ns;
+        a.out[1] = a.status ? *a.status : 0;
+    }
+    if (ns == 0 || ns == a.n) return;
+    const int base = b * kSplitPer + t * 4;
+    bool slow[4];
+    int cnt = 0;
+    for (int u = 0; u < 4; ++u) {
+        slow[u] = split_slow(a, base + u);
+        cnt += slow[u] ? 1 : 0;
+    }
+    lds[t] = cnt;
+    __syncthreads();
+    for (int off = 1; off < 256; off <<= 1) {
+        const int x = t >= off ? lds[t - off] : 0;
+        __syncthreads();
+        lds[t] += x;
+        __syncthreads();
+    }
+    int rank = before + lds[t] - cnt;  // slow particles before this one
+    const size_t n = static_cast<size_t>(a.n);
+    for (int u = 0; u < 4; ++u) {
+        const int i = base + u;
+        if (i >= a.n) break;
+        const int dst = slow[u] ? rank : ns + (i - rank);
+        if (slow[u]) ++rank;
+        for (int q = 0; q < a.narr; ++q) a.tmp[q * n + dst] = a.arr[q][i];
+    }
+}
+
+__global__ __launch_bounds__(256) void sia_split_copy_kernel(SplitArgs a)
+{
+    const int ns = a.out[0];
+    if (ns == 0 || ns == a.n) return;
+    const int i = static_cast<int>(blockIdx.x * 256u + threadIdx.x);
+    if (i >= a.n) return;
+    const size_t n = static_cast<size_t>(a.n);
+    for (int q = 0; q < a.narr; ++q) a.arr[q][i] = a.tmp[q * n + i];
+}
+
+struct UpdateArgs {
+    double* x[3];
+    const double* v[3];
+    long long* count;
+    double h;
+    int n;
+};
+
+// x += v h
+__global__ __launch_bounds__(256) void sia_axpy3_kernel(UpdateArgs a)
+{
+    const int i = static_cast<int>(blockIdx.x * 256u + threadIdx.x);
+    if (i >= a.n) return;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) a.x[d][i] = a.x[d][i] + a.v[d][i] * a.h;
+}
+
+// tstep = h, time += h, nstep += 1
+__global__ __launch_bounds__(256) void sia_book_kernel(UpdateArgs a)
+{
+    const int i = static_cast<int>(blockIdx.x * 256u + threadIdx.x);
+    if (i >= a.n) return;
+    a.x[0][i] = a.h;
+    a.x[1][i] = a.x[1][i] + a.h;
+    a.count[i] = a.count[i] + 1;
+}
+
+}  // namespace
+
+int sia_split_call(size_t n, void* const* arrays, int narrays, const double* tstep,
+                   double threshold, const int* status, int* out, void* stream)
+{
+    if (n < 1 || n > static_cast<size_t>(INT32_MAX))
+        return set_error(TUPAN_ERR_ARG, "particle count out of range");
+    if (narrays < 1 || narrays > kSplitArrays)
+        return set_error(TUPAN_ERR_ARG, "sia_split takes 1 to 32 arrays");
+    if (!arrays || !tstep || !out) return set_error(TUPAN_ERR_ARG, "null argument");
+    SplitArgs a{};
+    for (int q = 0; q < narrays; ++q) {
+        if (!arrays[q]) return set_error(TUPAN_ERR_ARG, "null array");
+        a.arr[q] = static_cast<unsigned long long*>(arrays[q]);
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const unsigned nb = static_cast<unsigned>((n + kSplitPer - 1) / kSplitPer);
+    const size_t b_tmp = (sizeof(unsigned long long) * narrays * n + 255) / 256 * 256;
+    char* w = static_cast<char*>(workspace(b_tmp + sizeof(int) * (nb + 64), s, 3));
+    if (!w) return set_error(TUPAN_ERR_ALLOC, "workspace allocation failed");
+    a.tmp = reinterpret_cast<unsigned long long*>(w);
+    a.out = reinterpret_cast<int*>(w + b_tmp);
+    a.blk = a.out + 64;
+    a.tstep = tstep;
+    a.status = status;
+    a.threshold = threshold;
+    a.n = static_cast<int>(n);
+    a.narr = narrays;
+    hipLaunchKernelGGL(sia_split_count_kernel, dim3(nb), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(sia_split_scatter_kernel, dim3(nb), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(sia_split_copy_kernel, dim3(static_cast<unsigned>((n + 255) / 256)),
+                       dim3(256), 0, s, a);
+    int rc = check_launch("sia_split");
+    if (rc == TUPAN_OK)
+        rc = check_hip(hipMemcpyAsync(out, a.out, 2 * sizeof(int), hipMemcpyDeviceToHost, s),
+                       "sia_split count");
+    if (rc == TUPAN_OK) rc = check_hip(hipStreamSynchronize(s), "sia_split count");
+    return rc;
+}
+
+int sia_update_call(int kind, size_t n, void* const* arrays, double h, void* stream)
+{
+    if (n > static_cast<size_t>(INT32_MAX))
+        return set_error(TUPAN_ERR_ARG, "particle count exceeds 2^31-1");
+    if (kind != 0 && kind != 1) return set_error(TUPAN_ERR_ARG, "unknown update");
+    if (!arrays) return set_error(TUPAN_ERR_ARG, "null argument");
+    for (int q = 0; q < (kind == 0 ? 6 : 3); ++q)
+        if (!arrays[q] && n > 0) return set_error(TUPAN_ERR_ARG, "null array");
+    if (n == 0) return TUPAN_OK;
+    UpdateArgs a{};
+    a.n = static_cast<int>(n);
+    a.h = h;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+    if (kind == 0) {
+        for (int d = 0; d < 3; ++d) {
+            a.x[d] = static_cast<double*>(arrays[d]);
+            a.v[d] = static_cast<const double*>(arrays[3 + d]);
+        }
+        hipLaunchKernelGGL(sia_axpy3_kernel, grid, dim3(256), 0, s, a);
+    } else {
+        a.x[0] = static_cast<double*>(arrays[0]);
+        a.x[1] = static_cast<double*>(arrays[1]);
+        a.count = static_cast<long long*>(arrays[2]);
+        hipLaunchKernelGGL(sia_book_kernel, grid, dim3(256), 0, s, a);
+    }
+    return check_launch("sia_update");
+}
+
+}  // namespace tupan
+
+// ===========================================================================
 // Device-scheduled hierarchical SIA steps (the 'h' variants,
 // sia.py:1089-1123), with no host read of level sizes.
 //

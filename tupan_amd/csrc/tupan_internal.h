@@ -169,6 +169,11 @@ int sia_subtree_call(int n, void* const* arrays, int narrays, const int* roles, 
                      const double* evolve_c, double* t_curr, unsigned long long* pairs,
                      int* status, void* stream);
 
+// Level operations of the host-driven hierarchical steps (sia.hip).
+int sia_split_call(size_t n, void* const* arrays, int narrays, const double* tstep,
+                   double threshold, const int* status, int* out, void* stream);
+int sia_update_call(int kind, size_t n, void* const* arrays, double h, void* stream);
+
 // Kepler-guess network (mlp.hip).  mlp_infer: delta[k] for the features
 // feat[4][n] (SoA) with the packed BF16 network `net`.
 int mlp_infer(int n, const float* feat, const void* net, float* delta, hipStream_t stream);

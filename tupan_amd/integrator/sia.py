@@ -108,6 +108,68 @@ def split(ps, condition):
     return slow, fast
 
 
+def _on_current_device(t):
+    return t.is_cuda and t.get_device() == torch.cuda.current_device()
+
+
+def _device_update(kind, tensors, h):
+    """tupan_sia_update on contiguous 8-byte arrays of one size on the
+    current device; False where they are not that (the caller then runs the same operations
+    array by array)."""
+    n = tensors[0].numel()
+    if not _on_current_device(tensors[0]):
+        return False
+    for t in tensors:
+        if not (t.is_cuda and t.element_size() == 8 and t.is_contiguous()
+                and t.numel() == n and not t.requires_grad):
+            return False
+    if kind == 0 and any(t.dtype != torch.float64 for t in tensors):
+        return False
+    from .. import _native
+    from ..lib.hip_backend import current_stream_handle
+    _native.check(_native.lib().tupan_sia_update(
+        kind, n, _native.ptr_array([t.data_ptr() for t in tensors]), h,
+        current_stream_handle()), "tupan_sia_update")
+    return True
+
+
+def _slow_count(ps, tstep, threshold, status=None):
+    """Partition ps's range of every array in place with tupan_sia_split and
+    return (slow particles, status word); None where the arrays are not
+    contiguous 8-byte device arrays."""
+    arrays = list(ps.arrays().values())
+    n = ps.n
+    if len(arrays) > 32 or tstep.dtype != torch.float64 \
+            or not _on_current_device(tstep):
+        return None
+    for t in arrays:
+        if not (t.is_cuda and t.element_size() == 8 and t.is_contiguous()
+                and t.numel() == n and not t.requires_grad):
+            return None
+    from .. import _native
+    from ..lib.hip_backend import current_stream_handle
+    out = (ctypes.c_int * 2)()
+    _native.check(_native.lib().tupan_sia_split(
+        n, _native.ptr_array([t.data_ptr() for t in arrays]), len(arrays),
+        tstep.data_ptr(), threshold,
+        None if status is None else status.data_ptr(), out,
+        current_stream_handle()), "tupan_sia_split")
+    return out[0], out[1]
+
+
+def partition_level(ps, threshold, subtree=None):
+    """``partition`` of ps by |tstep| > threshold; with the subtree helper of
+    the step, also the check of its status word so far."""
+    if ps.n > 2:
+        got = _slow_count(ps, ps.tstep, threshold,
+                          None if subtree is None else subtree.status)
+        if got is not None:
+            if subtree is not None:
+                subtree.check(got[1])
+            return ps[0:got[0]], ps[got[0]:ps.n]
+    return partition(ps, abs(ps.tstep) > threshold)
+
+
 def partition(ps, condition):
     """In-place form of ``split``: stably permute ps's range of every array
     to [slow | fast] and return slice views of the two parts.  ``ps`` must
@@ -136,18 +198,22 @@ def join(slow, fast):
 
 def drift(ips, tau):
     """sia.py:162-171 with drift_n and drift_pn (sia.py:64-101)."""
-    ips.rx += ips.vx * tau
-    ips.ry += ips.vy * tau
-    ips.rz += ips.vz * tau
+    if not _device_update(0, (ips.rx, ips.ry, ips.rz, ips.vx, ips.vy, ips.vz),
+                          tau):
+        ips.rx += ips.vx * tau
+        ips.ry += ips.vy * tau
+        ips.rz += ips.vz * tau
     if ips.include_pn_corrections:
         ips.pn_drift_com_r(tau)
     return ips
 
 
 def kick_n(ips, tau):
-    ips.vx += ips.ax * tau
-    ips.vy += ips.ay * tau
-    ips.vz += ips.az * tau
+    if not _device_update(0, (ips.vx, ips.vy, ips.vz, ips.ax, ips.ay, ips.az),
+                          tau):
+        ips.vx += ips.ax * tau
+        ips.vy += ips.ay * tau
+        ips.vz += ips.az * tau
     return ips
 
 
@@ -379,7 +445,13 @@ class SIA(Base):
         # worldline samples are taken
         self._subtree = (None if self.dumpper
                          else _DeviceSubtree.make(self, ps))
-        return self.recurse(ps, tau, self.evolve_set, self.scheme.bridge_sf)
+        if self._subtree is None:
+            return self.recurse(ps, tau, self.evolve_set,
+                                self.scheme.bridge_sf)
+        self._subtree.begin(ps)
+        ps = self.recurse(ps, tau, self.evolve_set, self.scheme.bridge_sf)
+        self._subtree.end(ps)
+        return ps
 
     def recurse(self, ps, tau, evolve, bridge_sf):
         """sia.py:1089-1123."""
@@ -395,15 +467,21 @@ class SIA(Base):
             ps.set_tstep(ps, self.eta)
             if self.shared_tstep:
                 tau = self.get_min_block_tstep(ps, tau)
-        cond = abs(ps.tstep) > flag * abs(tau)
-        slow, fast = (partition if self.inplace else split)(ps, cond)
+        if self.inplace:
+            slow, fast = partition_level(ps, flag * abs(tau), sub)
+        else:
+            slow, fast = split(ps, abs(ps.tstep) > flag * abs(tau))
         slow, fast = bridge_sf(slow, fast, tau, evolve, self.recurse)
         if fast.n == 0:
-            type(ps).t_curr += tau
+            if sub is not None:
+                sub.t_curr += tau
+            else:
+                type(ps).t_curr += tau
         if slow.n:
-            slow.tstep[...] = tau
-            slow.time += tau
-            slow.nstep += 1
+            if not _device_update(1, (slow.tstep, slow.time, slow.nstep), tau):
+                slow.tstep[...] = tau
+                slow.time += tau
+                slow.nstep += 1
             self.record_worldline(slow, tau)
         return ps if self.inplace else join(slow, fast)
 
@@ -744,20 +822,40 @@ class _DeviceSubtree(object):
         self.pairs = torch.zeros(2, dtype=torch.int64, device=device)
         self.status = torch.zeros(1, dtype=torch.int32, device=device)
 
-    def run(self, ps, tau):
-        from .. import _native
-        from ..lib import extensions
-        from ..lib.hip_backend import current_stream_handle
-        arrays = ps.arrays()
-        names = list(arrays)
-        ptrs = _native.ptr_array([t.data_ptr() for t in arrays.values()])
-        roles = (ctypes.c_int * len(SUBTREE_ROLES))(
+    def begin(self, ps):
+        """The step's start: the time, and cleared counters and status.  The
+        time is advanced on the device until end()."""
+        names = list(ps.arrays())
+        self.roles = (ctypes.c_int * len(SUBTREE_ROLES))(
             *[names.index(r) for r in SUBTREE_ROLES])
         self.t_curr.fill_(type(ps).t_curr)
         self.pairs.zero_()
         self.status.zero_()
+
+    def check(self, status):
+        if status:
+            from .. import _native
+            raise _native.TupanHipError(
+                "SIA subtree failed (status %d: 1 Kepler solver, 2 more than "
+                "64 levels, 3 more than 65536 level visits)" % status)
+
+    def end(self, ps):
+        """The step's end: the new time and the interactions counted."""
+        from ..lib import extensions
+        self.check(int(self.status.item()))
+        type(ps).t_curr = float(self.t_curr.item())
+        if extensions.pair_counts is not None:
+            tp, ap = self.pairs.tolist()
+            extensions.pair_counts["Tstep"] += tp
+            extensions.pair_counts["Acc"] += ap
+
+    def run(self, ps, tau):
+        from .. import _native
+        from ..lib.hip_backend import current_stream_handle
+        arrays = ps.arrays()
         rc = self.lib.tupan_sia_subtree(
-            ps.n, ptrs, len(names), ctypes.addressof(roles), self.modes[0],
+            ps.n, _native.ptr_array([t.data_ptr() for t in arrays.values()]),
+            len(arrays), ctypes.addressof(self.roles), self.modes[0],
             self.modes[1], self.sia.eta, tau, len(self.bridge_c),
             ctypes.addressof(self.bridge_op), ctypes.addressof(self.bridge_c),
             len(self.evolve_c), ctypes.addressof(self.evolve_op),
@@ -765,14 +863,4 @@ class _DeviceSubtree(object):
             self.pairs.data_ptr(), self.status.data_ptr(),
             current_stream_handle())
         _native.check(rc, "tupan_sia_subtree")
-        status = int(self.status.item())
-        if status:
-            raise _native.TupanHipError(
-                "SIA subtree failed (status %d: 1 Kepler solver, 2 more than "
-                "64 levels, 3 more than 65536 level visits)" % status)
-        type(ps).t_curr = float(self.t_curr.item())
-        if extensions.pair_counts is not None:
-            tp, ap = self.pairs.tolist()
-            extensions.pair_counts["Tstep"] += tp
-            extensions.pair_counts["Acc"] += ap
         return ps
