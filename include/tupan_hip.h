@@ -494,7 +494,9 @@ int tupan_sia_subtree(int n, void *const *arrays, int narrays, const int *roles,
  *
  * tupan_sia_update: kind 0, arrays {x0, x1, x2, v0, v1, v2}: x += v h;
  * kind 1, arrays {tstep, time, nstep (int64)}: tstep = h, time += h,
- * nstep += 1. */
+ * nstep += 1; kind 2, arrays as kind 0: x += (v h) / 2; kind 3, arrays
+ * {x0 .. x5, d0 .. d5}: x += d.  Kinds 2 and 3 are the Sakura drivers'
+ * (tupan/integrator/sakura.py:22-50). */
 int tupan_sia_split(size_t n, void *const *arrays, int narrays,
                     const double *tstep, double threshold, const int *status,
                     int *out, void *stream);

@@ -49,13 +49,14 @@ def test_partition_matches_array_operations(n, threshold):
 @pytest.mark.parametrize("n", [1, 255, 257, 70001])
 def test_updates_match_array_operations(n):
     from tupan_amd.integrator import sia
+    from tupan_amd.integrator.device_update import BOOK, device_update
     ps = system(n, 3, 1)
     other = ps.copy()
     a, b = ps[1:1 + n], other[1:1 + n]
     h = 0.1 / 3
     sia.drift(a, h)
     sia.kick_n(a, -h)
-    assert sia._device_update(1, (a.tstep, a.time, a.nstep), h)
+    assert device_update(BOOK, (a.tstep, a.time, a.nstep), h)
     for x, v in (("rx", "vx"), ("ry", "vy"), ("rz", "vz")):
         t = getattr(b, x)
         t += getattr(b, v) * h
@@ -68,11 +69,31 @@ def test_updates_match_array_operations(n):
     same(ps, other)
 
 
+@pytest.mark.parametrize("n", [1, 256, 70001])
+def test_sakura_updates_match_array_operations(n):
+    from tupan_amd.integrator import device_update as du
+    ps = system(n, 4, 0)
+    for k in ("drx", "dry", "drz", "dvx", "dvy", "dvz"):
+        ps.register_auxiliary_attribute(k, "real")
+        getattr(ps, k).copy_(ps.rx * 0.3 + ps.vy)
+    other = ps.copy()
+    tau = 0.1 / 3
+    du.half_drift(ps, tau)
+    du.apply_pair_drift(ps)
+    for x in "xyz":
+        t = getattr(other, "r" + x)
+        t += getattr(other, "v" + x) * tau / 2
+    for k in ("rx", "ry", "rz", "vx", "vy", "vz"):
+        t = getattr(other, k)
+        t += getattr(other, "d" + k)
+    same(ps, other)
+
+
 def test_other_arrays_keep_the_array_operations():
-    from tupan_amd.integrator import sia
+    from tupan_amd.integrator.device_update import DRIFT, device_update
     x = [torch.ones(8, device="cuda:0") for _ in range(6)]
-    assert not sia._device_update(0, x, 0.5)
+    assert not device_update(DRIFT, x, 0.5)
     y = [torch.ones(16, dtype=torch.float64, device="cuda:0")[::2]
          for _ in range(6)]
-    assert not sia._device_update(0, y, 0.5)
-    assert not sia._device_update(0, [t.cpu() for t in y], 0.5)
+    assert not device_update(DRIFT, y, 0.5)
+    assert not device_update(DRIFT, [t.cpu() for t in y], 0.5)

@@ -593,20 +593,33 @@ __global__ __launch_bounds__(256) void sia_split_copy_kernel(SplitArgs a)
 }
 
 struct UpdateArgs {
-    double* x[3];
-    const double* v[3];
+    double* x[6];
+    const double* v[6];
     long long* count;
     double h;
     int n;
 };
 
-// x += v h
+// x += v h, or x += (v h) / 2
+template <bool kHalf>
 __global__ __launch_bounds__(256) void sia_axpy3_kernel(UpdateArgs a)
 {
     const int i = static_cast<int>(blockIdx.x * 256u + threadIdx.x);
     if (i >= a.n) return;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) a.x[d][i] = a.x[d][i] + a.v[d][i] * a.h;
+    for (int d = 0; d < 3; ++d) {
+        const double vh = a.v[d][i] * a.h;
+        a.x[d][i] = a.x[d][i] + (kHalf ? vh * 0.5 : vh);
+    }
+}
+
+// six arrays x += v
+__global__ __launch_bounds__(256) void sia_add6_kernel(UpdateArgs a)
+{
+    const int i = static_cast<int>(blockIdx.x * 256u + threadIdx.x);
+    if (i >= a.n) return;
+#pragma unroll
+    for (int d = 0; d < 6; ++d) a.x[d][i] = a.x[d][i] + a.v[d][i];
 }
 
 // tstep = h, time += h, nstep += 1
@@ -663,9 +676,10 @@ int sia_update_call(int kind, size_t n, void* const* arrays, double h, void* str
 {
     if (n > static_cast<size_t>(INT32_MAX))
         return set_error(TUPAN_ERR_ARG, "particle count exceeds 2^31-1");
-    if (kind != 0 && kind != 1) return set_error(TUPAN_ERR_ARG, "unknown update");
+    constexpr int kArrays[4] = {6, 3, 6, 12};
+    if (kind < 0 || kind > 3) return set_error(TUPAN_ERR_ARG, "unknown update");
     if (!arrays) return set_error(TUPAN_ERR_ARG, "null argument");
-    for (int q = 0; q < (kind == 0 ? 6 : 3); ++q)
+    for (int q = 0; q < kArrays[kind]; ++q)
         if (!arrays[q] && n > 0) return set_error(TUPAN_ERR_ARG, "null array");
     if (n == 0) return TUPAN_OK;
     UpdateArgs a{};
@@ -673,18 +687,24 @@ int sia_update_call(int kind, size_t n, void* const* arrays, double h, void* str
     a.h = h;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 grid(static_cast<unsigned>((n + 255) / 256));
-    if (kind == 0) {
-        for (int d = 0; d < 3; ++d) {
-            a.x[d] = static_cast<double*>(arrays[d]);
-            a.v[d] = static_cast<const double*>(arrays[3 + d]);
-        }
-        hipLaunchKernelGGL(sia_axpy3_kernel, grid, dim3(256), 0, s, a);
-    } else {
+    if (kind == 1) {
         a.x[0] = static_cast<double*>(arrays[0]);
         a.x[1] = static_cast<double*>(arrays[1]);
         a.count = static_cast<long long*>(arrays[2]);
         hipLaunchKernelGGL(sia_book_kernel, grid, dim3(256), 0, s, a);
+        return check_launch("sia_update");
     }
+    const int m = kArrays[kind] / 2;
+    for (int d = 0; d < m; ++d) {
+        a.x[d] = static_cast<double*>(arrays[d]);
+        a.v[d] = static_cast<const double*>(arrays[m + d]);
+    }
+    if (kind == 0)
+        hipLaunchKernelGGL(sia_axpy3_kernel<false>, grid, dim3(256), 0, s, a);
+    else if (kind == 2)
+        hipLaunchKernelGGL(sia_axpy3_kernel<true>, grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL(sia_add6_kernel, grid, dim3(256), 0, s, a);
     return check_launch("sia_update");
 }
 

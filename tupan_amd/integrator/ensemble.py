@@ -12,6 +12,8 @@ steps run the same kernels in the same order as ``step``, so the results are
 the same numbers."""
 import torch
 
+from .device_update import apply_pair_drift, half_drift
+
 
 class SakuraEnsemble(object):
     def __init__(self, ps, ensemble):
@@ -28,21 +30,11 @@ class SakuraEnsemble(object):
     def _advance(self, tau, check):
         ps = self.ps
         ens = self.ens
-        ps.rx += ps.vx * tau / 2
-        ps.ry += ps.vy * tau / 2
-        ps.rz += ps.vz * tau / 2
+        half_drift(ps, tau)
         for flag in (-1, 1):
-            drx, dry, drz, dvx, dvy, dvz = ens.sakura(ps, tau / 2, flag,
-                                                      check=check)
-            ps.rx += drx
-            ps.ry += dry
-            ps.rz += drz
-            ps.vx += dvx
-            ps.vy += dvy
-            ps.vz += dvz
-        ps.rx += ps.vx * tau / 2
-        ps.ry += ps.vy * tau / 2
-        ps.rz += ps.vz * tau / 2
+            ens.sakura(ps, tau / 2, flag, check=check)
+            apply_pair_drift(ps)
+        half_drift(ps, tau)
 
     def evolve(self, t_end, tau):
         while self.time < t_end - 0.5 * abs(tau):

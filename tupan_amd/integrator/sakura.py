@@ -14,33 +14,16 @@ Sakura.evolve can replay a HIP graph of many steps.
 import torch
 
 from . import Base
+from .device_update import apply_pair_drift, half_drift
 from ..lib import extensions
 
 
 def sakura_step(ps, tau):
-    ps.rx += ps.vx * tau / 2
-    ps.ry += ps.vy * tau / 2
-    ps.rz += ps.vz * tau / 2
-
-    extensions.sakura.calc(ps, ps, tau / 2, -1)
-    ps.rx += ps.drx
-    ps.ry += ps.dry
-    ps.rz += ps.drz
-    ps.vx += ps.dvx
-    ps.vy += ps.dvy
-    ps.vz += ps.dvz
-
-    extensions.sakura.calc(ps, ps, tau / 2, 1)
-    ps.rx += ps.drx
-    ps.ry += ps.dry
-    ps.rz += ps.drz
-    ps.vx += ps.dvx
-    ps.vy += ps.dvy
-    ps.vz += ps.dvz
-
-    ps.rx += ps.vx * tau / 2
-    ps.ry += ps.vy * tau / 2
-    ps.rz += ps.vz * tau / 2
+    half_drift(ps, tau)
+    for flag in (-1, 1):
+        extensions.sakura.calc(ps, ps, tau / 2, flag)
+        apply_pair_drift(ps)
+    half_drift(ps, tau)
     return ps
 
 

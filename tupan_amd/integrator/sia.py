@@ -48,6 +48,7 @@ import logging
 import torch
 
 from . import Base
+from .device_update import device_update, on_current_device
 from .fewbody import FewBody
 
 SUBTREE_MAX = 64
@@ -108,31 +109,6 @@ def split(ps, condition):
     return slow, fast
 
 
-def _on_current_device(t):
-    return t.is_cuda and t.get_device() == torch.cuda.current_device()
-
-
-def _device_update(kind, tensors, h):
-    """tupan_sia_update on contiguous 8-byte arrays of one size on the
-    current device; False where they are not that (the caller then runs the same operations
-    array by array)."""
-    n = tensors[0].numel()
-    if not _on_current_device(tensors[0]):
-        return False
-    for t in tensors:
-        if not (t.is_cuda and t.element_size() == 8 and t.is_contiguous()
-                and t.numel() == n and not t.requires_grad):
-            return False
-    if kind == 0 and any(t.dtype != torch.float64 for t in tensors):
-        return False
-    from .. import _native
-    from ..lib.hip_backend import current_stream_handle
-    _native.check(_native.lib().tupan_sia_update(
-        kind, n, _native.ptr_array([t.data_ptr() for t in tensors]), h,
-        current_stream_handle()), "tupan_sia_update")
-    return True
-
-
 def _slow_count(ps, tstep, threshold, status=None):
     """Partition ps's range of every array in place with tupan_sia_split and
     return (slow particles, status word); None where the arrays are not
@@ -140,7 +116,7 @@ def _slow_count(ps, tstep, threshold, status=None):
     arrays = list(ps.arrays().values())
     n = ps.n
     if len(arrays) > 32 or tstep.dtype != torch.float64 \
-            or not _on_current_device(tstep):
+            or not on_current_device(tstep):
         return None
     for t in arrays:
         if not (t.is_cuda and t.element_size() == 8 and t.is_contiguous()
@@ -198,7 +174,7 @@ def join(slow, fast):
 
 def drift(ips, tau):
     """sia.py:162-171 with drift_n and drift_pn (sia.py:64-101)."""
-    if not _device_update(0, (ips.rx, ips.ry, ips.rz, ips.vx, ips.vy, ips.vz),
+    if not device_update(0, (ips.rx, ips.ry, ips.rz, ips.vx, ips.vy, ips.vz),
                           tau):
         ips.rx += ips.vx * tau
         ips.ry += ips.vy * tau
@@ -209,7 +185,7 @@ def drift(ips, tau):
 
 
 def kick_n(ips, tau):
-    if not _device_update(0, (ips.vx, ips.vy, ips.vz, ips.ax, ips.ay, ips.az),
+    if not device_update(0, (ips.vx, ips.vy, ips.vz, ips.ax, ips.ay, ips.az),
                           tau):
         ips.vx += ips.ax * tau
         ips.vy += ips.ay * tau
@@ -478,7 +454,7 @@ class SIA(Base):
             else:
                 type(ps).t_curr += tau
         if slow.n:
-            if not _device_update(1, (slow.tstep, slow.time, slow.nstep), tau):
+            if not device_update(1, (slow.tstep, slow.time, slow.nstep), tau):
                 slow.tstep[...] = tau
                 slow.time += tau
                 slow.nstep += 1
