@@ -11,9 +11,9 @@
 // back in place (the SIA n = 2 leaves, integrator/fewbody.py:30-42).
 //
 // Compiled with -ffp-contract=off (reference operation order).
-#include "engine.h"
 #include "kepler.h"
 #include "mlp_wave.h"
+#include "sym.h"
 #include "tupan_internal.h"
 
 namespace tupan {
@@ -30,11 +30,15 @@ struct SakuraArgs {
     unsigned long long* counters;
     int* status;
     // two-pass form (null in the one-pass form): per (j-split, i) the count
-    // of deferred near pairs and their j indices (kNearSlots slots each)
+    // of deferred near pairs and their j indices (near_slots slots each)
     int* near_count;
     int* near_j;
     // when set, dt is read from device memory (device-driven steps)
     const double* dt_dev;
+    int near_slots;  // list slots per entry
+    // symmetric far pass: blocks of the set and particles per block (0: the
+    // tile form, whose entry (s, i) covers the j-range of split s)
+    int nb, bi;
 };
 
 __device__ __forceinline__ double sakura_dt(const SakuraArgs& a)
@@ -42,9 +46,16 @@ __device__ __forceinline__ double sakura_dt(const SakuraArgs& a)
     return a.dt_dev ? *a.dt_dev : a.dt;
 }
 
-// Near pairs listed per (j-split, i); further ones are solved by
-// near_overflow_kernel.
+// Near pairs listed per entry; entries with more are solved by
+// near_overflow_kernel.  An entry is an i and the partners one wave met it
+// with: a j-split in the tile form, fewer in the symmetric form.
 constexpr int kNearSlots = 32;
+constexpr int kNearSlotsSym = 8;
+
+__device__ __forceinline__ int near_listed(int count, int slots)
+{
+    return count > slots ? 0 : count;
+}
 // Calls with at least this many pairs take the two-pass form by default.
 constexpr double kTwoPassPairs = 4194304.0;
 // i-particles per thread in the far-pair pass (independent dependency
@@ -261,7 +272,7 @@ __global__ __launch_bounds__(BLOCK) void sakura_far_kernel(SakuraArgs a)
         Op::load_i(a, {}, valid[w] ? i : a.ni - 1, r[w]);
         Op::zero(acc[w]);
         const size_t entry = static_cast<size_t>(g.jsplit) * a.ni + (valid[w] ? i : 0);
-        slots[w] = a.near_j + entry * kNearSlots;
+        slots[w] = a.near_j + entry * a.near_slots;
         ndef[w] = 0;
     }
     const int j0 = g.jsplit * a.jchunk;
@@ -283,9 +294,9 @@ __global__ __launch_bounds__(BLOCK) void sakura_far_kernel(SakuraArgs a)
                 double p[3] = {p0[0], p0[1], p0[2]};
                 double v[3] = {v0[0], v0[1], v0[2]};
                 if (!kep::drift_twobody_far_t<FLAG>(r[w].dt, m, e2, p, v, acc[w].c)) {
-                    // near pair: the first kNearSlots go to the list, the
-                    // rest to near_overflow_kernel
-                    if (ndef[w] < kNearSlots) slots[w][ndef[w]] = jt + k;
+                    // near pair; an entry with more than its slots goes to
+                    // near_overflow_kernel whole
+                    if (ndef[w] < a.near_slots) slots[w][ndef[w]] = jt + k;
                     ++ndef[w];
                     continue;
                 }
@@ -316,7 +327,174 @@ __global__ __launch_bounds__(BLOCK) void sakura_far_kernel(SakuraArgs a)
     if (a.status && tot.fail) atomicOr(a.status, 1);
 }
 
-// Exclusive scan of the listed counts min(count, kNearSlots) in three
+// The far pass of a set against itself, each unordered pair once (sym.h has
+// the decomposition and the rotation; here one wave holds a block, W of its
+// particles a lane's, so the near lists fill in a fixed order).  The
+// relative orbit of j about i is i's about j mirrored: the far/near test and
+// the increments are the same numbers, so a pair costs its drift once and six
+// weighted sums per side, 140 instructions for the two where the tile form
+// takes 2 x 126.  A near pair goes to both particles' entries: (chunk, i),
+// and (nchunk + d - 1, j) for a row d blocks away, whose count moves with the
+// j sums.  Entry sums and counts are all written: for an even block count the
+// upper rows, which have no partner at the last distance, write its zeros.
+// The waves of a workgroup are independent tasks, four to a workgroup so that
+// every SIMD gets one (workgroups of a single wave left SIMDs with two and
+// others with none: 1.12 ms at N = 16384 for the same plan).  Whole call,
+// flag -1: N = 16384 1.26 -> 0.84 ms, 65536 19.4 -> 9.5 ms.
+constexpr int kSymFarWaves = 4;
+
+// LDS written and read by one wave alone: its accesses happen in order, the
+// compiler is told to keep them so.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int W, long FLAG>
+__global__ __launch_bounds__(kWave* kSymFarWaves, 2) void sakura_far_sym_kernel(SakuraArgs a)
+{
+    using Op = OpSakura;
+    constexpr int BI = kWave * W;
+    constexpr int F = 8;
+    __shared__ double slots[kSymFarWaves][F * 2 * kWave];
+    const int n = a.ni;
+    const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+    const int wave = static_cast<int>(threadIdx.x) / kWave;
+    double* slot = slots[wave];
+    const int nchunk = a.nsplit - a.nb / 2;
+    const int task = static_cast<int>(blockIdx.x) * kSymFarWaves + wave;
+    const int row = task / nchunk;
+    const int chunk = task % nchunk;
+    if (row >= a.nb) return;
+    const double dt = sakura_dt(a);
+    Op::Slot I[W];
+    double acc[W][6];
+    int ndef[W];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        const int i = row * BI + w * kWave + lane;
+        Op::load_j(a, {}, i < n ? i : n - 1, I[w]);
+        ndef[w] = 0;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) acc[w][k] = 0.0;
+    }
+    const int tiles = sym_row_tiles(a.nb, row, W);
+    const int t0 = static_cast<int>(static_cast<long long>(tiles) * chunk / nchunk);
+    const int t1 = static_cast<int>(static_cast<long long>(tiles) * (chunk + 1) / nchunk);
+    kep::Counters tot;
+    for (int t = t0; t < t1; ++t) {
+        const int d = t / W;
+        int block = row + d;
+        if (block >= a.nb) block -= a.nb;
+        const int j0 = block * BI + (t % W) * kWave;
+        if (j0 >= n) continue;
+        const int jn = min(kWave, n - j0);
+        wave_lds_sync();
+        {
+            Op::Slot s;
+            Op::load_j(a, {}, lane < jn ? j0 + lane : n - 1, s);
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                slot[f * 2 * kWave + lane] = s.v[f];
+                slot[f * 2 * kWave + kWave + lane] = s.v[f];
+            }
+        }
+        wave_lds_sync();
+        const size_t jentry = static_cast<size_t>(nchunk + d - 1) * n + j0;
+        double aj[6] = {0, 0, 0, 0, 0, 0};
+        int jdef = 0;
+        kep::Counters c;
+        for (int s = 0; s < kWave; ++s) {
+            const double* base = slot + kWave - s + lane;
+            double J[F];
+#pragma unroll
+            for (int f = 0; f < F; ++f) J[f] = base[f * 2 * kWave];
+            const int jl = (lane - s) & (kWave - 1);
+            wave_ror1(aj);
+            jdef = __builtin_amdgcn_update_dpp(jdef, jdef, 0x13C, 0xf, 0xf, false);
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const int i = row * BI + w * kWave + lane;
+                if (i >= n || jl >= jn) continue;
+                const double p0[3] = {I[w].v[1] - J[1], I[w].v[2] - J[2], I[w].v[3] - J[3]};
+                const double e2 = I[w].v[4] + J[4];
+                const double v0[3] = {I[w].v[5] - J[5], I[w].v[6] - J[6], I[w].v[7] - J[7]};
+                const double m = I[w].v[0] + J[0];
+                double p[3] = {p0[0], p0[1], p0[2]};
+                double v[3] = {v0[0], v0[1], v0[2]};
+                if (!kep::drift_twobody_far_t<FLAG>(dt, m, e2, p, v, c)) {
+                    if (ndef[w] < a.near_slots)
+                        a.near_j[(static_cast<size_t>(chunk) * n + i) * a.near_slots + ndef[w]] =
+                            j0 + jl;
+                    ++ndef[w];
+                    if (d > 0) {
+                        if (jdef < a.near_slots)
+                            a.near_j[(jentry + jl) * a.near_slots + jdef] = i;
+                        ++jdef;
+                    }
+                    continue;
+                }
+                const double rec = kep::recip_refined(m);
+                const double mu = J[0] * rec, nu = -(I[w].v[0] * rec);
+                const double g[6] = {p[0] - p0[0], p[1] - p0[1], p[2] - p0[2],
+                                     v[0] - v0[0], v[1] - v0[1], v[2] - v0[2]};
+#pragma unroll
+                for (int k = 0; k < 6; ++k) {
+                    acc[w][k] = __builtin_fma(mu, g[k], acc[w][k]);
+                    aj[k] = __builtin_fma(nu, g[k], aj[k]);
+                }
+            }
+        }
+        tot.leapfrog += d > 0 ? 2 * c.leapfrog : c.leapfrog;
+        // after the last step lane l holds particle l + 1
+        const int jl = (lane + 1) & (kWave - 1);
+        if (d > 0 && jl < jn) {
+            double* part = a.partial + static_cast<size_t>(nchunk + d - 1) * 6 * n + j0 + jl;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) part[static_cast<size_t>(k) * n] = aj[k];
+            a.near_count[jentry + jl] = jdef;
+        }
+    }
+    if (a.nb % 2 == 0 && row >= a.nb / 2 && chunk == nchunk - 1) {
+        const int j0 = (row - a.nb / 2) * BI;
+        for (int j = j0 + lane; j < min(n, j0 + BI); j += kWave) {
+            double* part = a.partial + static_cast<size_t>(a.nsplit - 1) * 6 * n + j;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) part[static_cast<size_t>(k) * n] = 0.0;
+            a.near_count[static_cast<size_t>(a.nsplit - 1) * n + j] = 0;
+        }
+    }
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        const int i = row * BI + w * kWave + lane;
+        if (i >= n) continue;
+        double* part = a.partial + static_cast<size_t>(chunk) * 6 * n + i;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) part[static_cast<size_t>(k) * n] = acc[w][k];
+        a.near_count[static_cast<size_t>(chunk) * n + i] = ndef[w];
+    }
+    flush_counters(a.counters, true, tot, lane);
+}
+
+constexpr int kFarBlock = 128, kFarTile = 64;
+
+template <long FLAG>
+static void launch_far(const SakuraArgs& a, unsigned grid, hipStream_t s)
+{
+    if (a.bi == 4 * kWave)
+        hipLaunchKernelGGL((sakura_far_sym_kernel<4, FLAG>), dim3(grid),
+                           dim3(kWave * kSymFarWaves), 0, s, a);
+    else if (a.bi == 2 * kWave)
+        hipLaunchKernelGGL((sakura_far_sym_kernel<2, FLAG>), dim3(grid),
+                           dim3(kWave * kSymFarWaves), 0, s, a);
+    else
+        hipLaunchKernelGGL((sakura_far_kernel<kFarBlock, kFarTile, kFarWpt, FLAG>), dim3(grid),
+                           dim3(kFarBlock), 0, s, a);
+}
+
+// Exclusive scan of the listed counts (near_listed) in three
 // kernels: per-block sums (kScanPer entries per block, each thread four
 // consecutive ones), a one-workgroup scan of the block sums, and the
 // per-block scan that writes the offsets.  total[0] receives the listed
@@ -344,7 +522,8 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* lds, int& block_
     return incl - v;
 }
 
-__global__ __launch_bounds__(kScanThreads) void near_block_sums_kernel(int n, const int* count,
+__global__ __launch_bounds__(kScanThreads) void near_block_sums_kernel(int n, int slots,
+                                                                       const int* count,
                                                                        int* bsum, int* bover)
 {
     __shared__ int lds[kScanThreads];
@@ -354,8 +533,8 @@ __global__ __launch_bounds__(kScanThreads) void near_block_sums_kernel(int n, co
         const int e = base + q;
         if (e < n) {
             const int c = count[e];
-            sum += min(c, kNearSlots);
-            ov += c > kNearSlots;
+            sum += near_listed(c, slots);
+            ov += c > slots;
         }
     }
     int tot_s, tot_o;
@@ -398,7 +577,8 @@ __global__ __launch_bounds__(kScanThreads) void near_block_offsets_kernel(int nb
     }
 }
 
-__global__ __launch_bounds__(kScanThreads) void near_offsets_kernel(int n, const int* count,
+__global__ __launch_bounds__(kScanThreads) void near_offsets_kernel(int n, int slots,
+                                                                    const int* count,
                                                                     const int* boff, int* off,
                                                                     int* total, int* over_list)
 {
@@ -409,7 +589,7 @@ __global__ __launch_bounds__(kScanThreads) void near_offsets_kernel(int n, const
     for (int q = 0; q < 4; ++q) {
         const int e = base + q;
         c[q] = e < n ? count[e] : 0;
-        sum += min(c[q], kNearSlots);
+        sum += near_listed(c[q], slots);
     }
     int tot;
     int run = boff[blockIdx.x] + block_exclusive_scan(sum, lds, tot);
@@ -417,25 +597,26 @@ __global__ __launch_bounds__(kScanThreads) void near_offsets_kernel(int n, const
         const int e = base + q;
         if (e >= n) break;
         off[e] = run;
-        run += min(c[q], kNearSlots);
-        if (c[q] > kNearSlots) over_list[atomicAdd(total + 2, 1)] = e;
+        run += near_listed(c[q], slots);
+        if (c[q] > slots) over_list[atomicAdd(total + 2, 1)] = e;
     }
 }
 
-// Near-pair list: item = (i, j), grouped by (split, i), j ascending.
+// Near-pair list: item = (i, partner), grouped by entry, in the order met.
 // Items at or beyond `cap` are not written (a call whose list is longer
 // than its capacity is flagged by near_capacity_kernel).
-__global__ __launch_bounds__(256) void near_compact_kernel(int n, int ni, const int* count,
-                                                           const int* off, const int* near_j,
+__global__ __launch_bounds__(256) void near_compact_kernel(int n, int ni, int slots,
+                                                           const int* count, const int* off,
+                                                           const int* near_j,
                                                            int2* items, int cap)
 {
     const int e = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= n) return;
-    const int c = min(count[e], kNearSlots);
+    const int c = near_listed(count[e], slots);
     const int o = off[e];
     const int i = e % ni;
     for (int k = 0; k < c && o + k < cap; ++k)
-        items[o + k] = make_int2(i, near_j[static_cast<size_t>(e) * kNearSlots + k]);
+        items[o + k] = make_int2(i, near_j[static_cast<size_t>(e) * slots + k]);
 }
 
 // Capacity check of the graph-safe form: status bit 2 when the near-pair
@@ -588,13 +769,13 @@ __global__ __launch_bounds__(128, 2) void sakura_near_learned_kernel(SakuraArgs 
 
 // Pass 3: add each (split, i)'s near contributions, in list order, to its
 // far partial sum.
-__global__ __launch_bounds__(256) void near_add_kernel(int n, int ni, int nitems,
+__global__ __launch_bounds__(256) void near_add_kernel(int n, int ni, int nitems, int slots,
                                                        const int* count, const int* off,
                                                        const double* contrib, double* partial)
 {
     const int e = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= n) return;
-    const int c = min(count[e], kNearSlots);
+    const int c = near_listed(count[e], slots);
     if (c == 0) return;
     const int o = off[e];
     const int split = e / ni;
@@ -608,25 +789,59 @@ __global__ __launch_bounds__(256) void near_add_kernel(int n, int ni, int nitems
     }
 }
 
+// The partners of an entry: how many candidates, and candidate k (a particle
+// index, or -1 where the last block ends).
+struct Partners {
+    int first, count;   // tile form and j entries: consecutive particles
+    int row, t0;        // i entries of the symmetric form: tiles from t0 on
+};
+
+__device__ __forceinline__ Partners entry_partners(const SakuraArgs& a, int split, int i)
+{
+    if (a.nb == 0) {
+        const int j0 = split * a.jchunk;
+        return {j0, min(a.nj, j0 + a.jchunk) - j0, -1, 0};
+    }
+    const int block = i / a.bi;
+    const int nchunk = a.nsplit - a.nb / 2;
+    if (split >= nchunk) {
+        int row = block - (split - nchunk + 1);
+        if (row < 0) row += a.nb;
+        return {row * a.bi, a.bi, -1, 0};
+    }
+    const int tiles = sym_row_tiles(a.nb, block, a.bi / kWave);
+    const int t0 = static_cast<int>(static_cast<long long>(tiles) * split / nchunk);
+    const int t1 = static_cast<int>(static_cast<long long>(tiles) * (split + 1) / nchunk);
+    return {0, (t1 - t0) * kWave, block, t0};
+}
+
+__device__ __forceinline__ int partner(const SakuraArgs& a, const Partners& P, int k)
+{
+    if (k >= P.count) return -1;
+    int j = P.first + k;
+    if (P.row >= 0) {
+        const int t = P.t0 + k / kWave, tpb = a.bi / kWave;
+        int block = P.row + t / tpb;
+        if (block >= a.nb) block -= a.nb;
+        j = block * a.bi + (t % tpb) * kWave + k % kWave;
+    }
+    return j < a.nj ? j : -1;
+}
+
 // Entries with more near pairs than list slots, one wave per entry: the
-// wave walks its j range in chunks of 64 (one j per lane), ranks the near
-// pairs of the chunk in j order with a ballot, solves those ranked after the
-// first kNearSlots (in parallel, one per lane), and adds the chunk's
-// contributions to the partial sum through a fixed shuffle tree
-// (deterministic).
+// wave walks the entry's partners in chunks of 64 (one per lane), solves the
+// near ones in parallel and adds the chunk's contributions to the partial
+// sum through a fixed shuffle tree (deterministic).
 __device__ __forceinline__ void overflow_entry(const SakuraArgs& a, int e, int lane,
                                                kep::Counters& c)
 {
     const int split = e / a.ni;
     const int i = e % a.ni;
-    const int j0 = split * a.jchunk;
-    const int j1 = min(a.nj, j0 + a.jchunk);
+    const Partners P = entry_partners(a, split, i);
     double d[6] = {0, 0, 0, 0, 0, 0};
-    int seen = 0;  // near pairs before this chunk
-    for (int jb = j0; jb < j1; jb += kWave) {
-        const int j = jb + lane;
-        const bool inr = j < j1;
-        const int jj = inr ? j : j0;
+    for (int kb = 0; kb < P.count; kb += kWave) {
+        const int j = partner(a, P, kb + lane);
+        const int jj = j < 0 ? i : j;
         const double p0[3] = {a.ip[1][i] - a.jp[1][jj], a.ip[2][i] - a.jp[2][jj],
                               a.ip[3][i] - a.jp[3][jj]};
         const double e2 = a.ip[4][i] + a.jp[4][jj];
@@ -637,12 +852,10 @@ __device__ __forceinline__ void overflow_entry(const SakuraArgs& a, int e, int l
         double p[3] = {p0[0], p0[1], p0[2]};
         double v[3] = {v0[0], v0[1], v0[2]};
         kep::Counters scratch;
-        const bool near = inr && !kep::drift_twobody_far(sakura_dt(a), a.flag, m, e2, p, v, scratch);
-        const unsigned long long mask = __ballot(near);
-        const int rank = seen + __popcll(mask & ((1ull << lane) - 1ull));
-        seen += __popcll(mask);
+        const bool near =
+            j >= 0 && !kep::drift_twobody_far(sakura_dt(a), a.flag, m, e2, p, v, scratch);
         double cd[6] = {0, 0, 0, 0, 0, 0};
-        if (near && rank >= kNearSlots) {
+        if (near) {
             p[0] = p0[0]; p[1] = p0[1]; p[2] = p0[2];
             v[0] = v0[0]; v[1] = v0[1]; v[2] = v0[2];
             kep::drift_twobody(sakura_dt(a), a.flag, m, e2, p, v, c);
@@ -683,6 +896,53 @@ __global__ __launch_bounds__(64) void near_overflow_kernel(SakuraArgs a, const i
     if (a.status && c.fail) atomicOr(a.status, 1);
 }
 
+// The symmetric far pass's plan for a set against itself; false where the
+// tile form takes the call: up to kSymFarAbove particles, where it spreads
+// the work finer (n = 4096: 244 us, 253 symmetric; 6000: 321 and 264 us), and
+// where the entries' sums, counts and lists pass kSymMaxBytes (n = 150000).
+// Four particles per lane above kSymFarW4Above (n = 12000: 543 us with four,
+// 498 with two; 24001: 1507 and 1556 us; 65536: 9.50 and 9.74 ms).  Chunks
+// per row: at least two waves per SIMD, and of the counts up to four times
+// that the one whose busiest SIMD has the least to do, a wave's fixed cost
+// counted as a quarter of a tile.
+constexpr int kSymFarAbove = 5120, kSymFarW4Above = 20480;
+
+static bool sakura_sym_plan(SakuraArgs& a, int cu, unsigned* grid)
+{
+    bool same = a.ni == a.nj;
+    for (int f = 0; f < 8; ++f) same = same && a.ip[f] == a.jp[f];
+    if (!same || a.ni <= kSymFarAbove) return false;
+    const int W = a.ni > kSymFarW4Above ? 4 : 2;
+    const int bi = kWave * W;
+    const int nb = (a.ni + bi - 1) / bi;
+    const int tiles = sym_row_tiles(nb, 0, W);
+    const int simds = 4 * cu;
+    int lo = (2 * simds + nb - 1) / nb;
+    if (lo > tiles) lo = tiles;
+    int nchunk = lo;
+    long long best = -1;
+    for (int nc = lo; nc <= tiles && nc <= 4 * lo; ++nc) {
+        const long long cost = ((static_cast<long long>(nb) * nc + simds - 1) / simds) *
+                               (4 * ((tiles + nc - 1) / nc) + 1);
+        if (best < 0 || cost < best) {
+            best = cost;
+            nchunk = nc;
+        }
+    }
+    const size_t slots = static_cast<size_t>(nchunk) + nb / 2;
+    const size_t nent = slots * a.ni;
+    constexpr size_t kEntryBytes = 6 * sizeof(double) + (3 + kNearSlotsSym) * sizeof(int);
+    if (nent * kEntryBytes > kSymMaxBytes) return false;
+    a.nb = nb;
+    a.bi = bi;
+    a.nsplit = static_cast<int>(slots);
+    a.jchunk = 0;
+    a.near_slots = kNearSlotsSym;
+    *grid = (static_cast<unsigned>(nb) * static_cast<unsigned>(nchunk) + kSymFarWaves - 1) /
+            kSymFarWaves;
+    return true;
+}
+
 int sakura_call(size_t ni, const double* const* ip, size_t nj, const double* const* jp,
                 double dt, long flag, double* const* out, unsigned long long* counters,
                 int* status, void* stream)
@@ -715,7 +975,7 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
     a.counters = counters;
     a.status = status;
     a.dt_dev = opt.dt_dev;
-    constexpr int BLOCK = 128, TILE = 64;
+    constexpr int BLOCK = kFarBlock, TILE = kFarTile;
     const Device& dev = current_device();
     hipStream_t s = static_cast<hipStream_t>(stream);
     bool two_pass = opt.path == 2 ||
@@ -741,8 +1001,10 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
     }
     a.nsplit = L.nsplit;
     a.jchunk = L.jchunk;
+    a.near_slots = kNearSlots;
     opt.near_pairs = -1;
-    const unsigned grid = static_cast<unsigned>(L.nblock_i) * static_cast<unsigned>(L.nsplit);
+    unsigned grid = static_cast<unsigned>(L.nblock_i) * static_cast<unsigned>(L.nsplit);
+    if (two_pass && sakura_sym_plan(a, dev.cu_count, &grid)) nent = static_cast<size_t>(a.nsplit) * ni;
     const unsigned rg = static_cast<unsigned>((a.ni + 255) / 256);
     if (!two_pass) {
         if (L.nsplit > 1) {
@@ -757,7 +1019,6 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
             hipLaunchKernelGGL((reduce_kernel<OpSakura>), dim3(rg), dim3(256), 0, s, a);
         return check_launch("sakura");
     }
-    const unsigned fgrid = grid;
 
     // workspace slot 1: partials [nsplit][6][ni], counts, offsets, the
     // overflow list, block sums, totals, the near pass's counter bank and
@@ -770,7 +1031,7 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
     const size_t b_blk = up(static_cast<size_t>(nb) * sizeof(int));
     const size_t b_tot = 256;
     const size_t b_bank = up(kBankSlots * kBankStride * sizeof(unsigned long long));
-    const size_t b_slots = up(nent * kNearSlots * sizeof(int));
+    const size_t b_slots = up(nent * a.near_slots * sizeof(int));
     char* w1 = static_cast<char*>(
         workspace(b_part + 3 * b_cnt + 2 * b_blk + b_tot + b_bank + b_slots, s, 1));
     if (!w1) return set_error(TUPAN_ERR_ALLOC, "workspace allocation failed");
@@ -798,36 +1059,21 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
     timing_begin(s);
     // the flag as a template argument: no flag tests in the pair loop
     switch (a.flag) {
-    case -1:
-        hipLaunchKernelGGL((sakura_far_kernel<BLOCK, TILE, kFarWpt, -1>), dim3(fgrid),
-                           dim3(BLOCK), 0, s, a);
-        break;
-    case 1:
-        hipLaunchKernelGGL((sakura_far_kernel<BLOCK, TILE, kFarWpt, 1>), dim3(fgrid),
-                           dim3(BLOCK), 0, s, a);
-        break;
-    case -2:
-        hipLaunchKernelGGL((sakura_far_kernel<BLOCK, TILE, kFarWpt, -2>), dim3(fgrid),
-                           dim3(BLOCK), 0, s, a);
-        break;
-    case 2:
-        hipLaunchKernelGGL((sakura_far_kernel<BLOCK, TILE, kFarWpt, 2>), dim3(fgrid),
-                           dim3(BLOCK), 0, s, a);
-        break;
-    default:
-        hipLaunchKernelGGL((sakura_far_kernel<BLOCK, TILE, kFarWpt, 0>), dim3(fgrid),
-                           dim3(BLOCK), 0, s, a);
-        break;
+    case -1: launch_far<-1>(a, grid, s); break;
+    case 1: launch_far<1>(a, grid, s); break;
+    case -2: launch_far<-2>(a, grid, s); break;
+    case 2: launch_far<2>(a, grid, s); break;
+    default: launch_far<0>(a, grid, s); break;
     }
     // timed as two intervals: the far-pair kernel, then the rest of the call
     timing_end(s);
     timing_begin(s);
     hipLaunchKernelGGL(near_block_sums_kernel, dim3(nb), dim3(kScanThreads), 0, s, n,
-                       a.near_count, bsum, bover);
+                       a.near_slots, a.near_count, bsum, bover);
     hipLaunchKernelGGL(near_block_offsets_kernel, dim3(1), dim3(kScanThreads), 0, s, nb, bsum,
                        bover, total_dev, bank);
     hipLaunchKernelGGL(near_offsets_kernel, dim3(nb), dim3(kScanThreads), 0, s, n,
-                       a.near_count, bsum, near_off, total_dev, over_list);
+                       a.near_slots, a.near_count, bsum, near_off, total_dev, over_list);
     const unsigned eg = static_cast<unsigned>((n + 255) / 256);
     if (graph) {
         // No host synchronisation: the list gets the caller's capacity, the
@@ -842,15 +1088,15 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
         int2* items = reinterpret_cast<int2*>(w2);
         double* contrib = reinterpret_cast<double*>(w2 + b_items);
         hipLaunchKernelGGL(near_capacity_kernel, dim3(1), dim3(64), 0, s, total_dev, cap, status);
-        hipLaunchKernelGGL(near_compact_kernel, dim3(eg), dim3(256), 0, s, n, a.ni, a.near_count,
-                           near_off, a.near_j, items, cap);
+        hipLaunchKernelGGL(near_compact_kernel, dim3(eg), dim3(256), 0, s, n, a.ni,
+                           a.near_slots, a.near_count, near_off, a.near_j, items, cap);
         hipLaunchKernelGGL(sakura_near_kernel, dim3((cap + 127) / 128), dim3(128), 0, s, a, cap,
                            total_dev, items, contrib, nullptr, opt.log, bank);
         if (bank)
             hipLaunchKernelGGL(near_bank_flush_kernel, dim3(1), dim3(64), 0, s, bank, a.counters,
                                opt.fallbacks);
         hipLaunchKernelGGL(near_add_kernel, dim3(eg), dim3(256), 0, s, n, a.ni, cap,
-                           a.near_count, near_off, contrib, a.partial);
+                           a.near_slots, a.near_count, near_off, contrib, a.partial);
         hipLaunchKernelGGL(near_overflow_kernel, dim3(kOverflowWaves), dim3(kWave), 0, s, a,
                            over_list, 0, total_dev + 1);
         hipLaunchKernelGGL((reduce_kernel<OpSakura>), dim3(rg), dim3(256), 0, s, a);
@@ -876,7 +1122,7 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
         int2* items = reinterpret_cast<int2*>(w2);
         double* contrib = reinterpret_cast<double*>(w2 + b_items);
         hipLaunchKernelGGL(near_compact_kernel, dim3(eg), dim3(256), 0, s, n, a.ni,
-                           a.near_count, near_off, a.near_j, items, total);
+                           a.near_slots, a.near_count, near_off, a.near_j, items, total);
         const unsigned ig = static_cast<unsigned>((total + 127) / 128);
         if (opt.net) {
             hipLaunchKernelGGL(sakura_near_learned_kernel, dim3(ig), dim3(128), 0, s, a, total,
@@ -890,7 +1136,7 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
             hipLaunchKernelGGL(near_bank_flush_kernel, dim3(1), dim3(64), 0, s, bank, a.counters,
                                opt.fallbacks);
         hipLaunchKernelGGL(near_add_kernel, dim3(eg), dim3(256), 0, s, n, a.ni, total,
-                           a.near_count, near_off, contrib, a.partial);
+                           a.near_slots, a.near_count, near_off, contrib, a.partial);
     }
     if (counts[1] > 0) {
         hipLaunchKernelGGL(near_overflow_kernel, dim3(counts[1]), dim3(kWave), 0, s, a,
