@@ -91,10 +91,12 @@ int tupan_timing_read_each(double *ms, int max, int *count);
  * table entry for (kernel TUPAN_K_*, slot, bucket) picks the shape and the
  * workgroups-per-CU target of the launch planner.  slot: 0 FP64, 1
  * split-FP32, 2 reference-order FP64, 3 float build.  bucket by pair count
- * ni*nj: 0 below 2^22, 1 below 2^30, 2 above.  Default: shape 0, 4
- * workgroups per CU.  The table is process-wide.  Calls of at most 2^21
- * pairs with 256 < nj <= 2048 (any mode but reference-order FP64) run a
- * one-launch small-set kernel that does not consult the table. */
+ * ni*nj: 0 below 2^25, 1 below 2^30, 2 above; a call whose ni the picked
+ * shape would pad by more than a quarter takes bucket 0's entry.  Default:
+ * shape 0, 4 workgroups per CU.  The table is process-wide.  Calls of at
+ * most 2^21 pairs with 256 < nj <= 2048 (any mode but reference-order FP64)
+ * run a one-launch small-set kernel that does not consult the table, and a
+ * set against itself above a few thousand particles the symmetric engine. */
 #define TUPAN_TUNE_SHAPES 6
 #define TUPAN_TUNE_BUCKETS 3
 int tupan_tune_set(int kernel, int slot, int bucket, int shape, int wg_per_cu);

@@ -47,3 +47,14 @@ def test_rows_vs_oracle(ni, nj, mode):
     w = (dj["mass"] * np.sqrt(r2) / (r2 + 2e-6)**1.5).sum(1)
     err = np.sqrt(sum((g - r)**2 for g, r in zip(got, ref)))
     assert np.max(err / w) <= 8 * 2.0**-24
+
+
+@pytest.mark.parametrize("mode", ["fp64", "split32", "ieee64"])
+@pytest.mark.parametrize("ni,nj", [(1024, 32767), (1024, 32768),
+                                   (300, 500001), (1025, 1048576),
+                                   (1300, 1048577), (1024, 1048575)])
+def test_bucket_edges_and_padded_rows_vs_oracle(ni, nj, mode):
+    """Both sides of the table's pair-count lines (2^25, 2^30) and sets whose
+    rows fill a quarter to nine tenths of the tuned shape's workgroup, which
+    take the one-wave shape: same tolerances."""
+    test_rows_vs_oracle(ni, nj, mode)

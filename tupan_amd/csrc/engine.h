@@ -499,9 +499,33 @@ __global__ __launch_bounds__(256) void fallback_kernel(typename Op::Args a)
 // Acc, AccJerk, Tstep, split forms); the last, one wave per workgroup, is
 // for small systems.  The tuning table picks one per kernel, mode and size.
 constexpr int kNumShapes = 6;
+constexpr int kNumBuckets = 3;
 constexpr int kLightShapeDims[kNumShapes][4] = {
     {256, 2, 256, 4}, {512, 2, 512, 2}, {256, 4, 256, 2}, {128, 2, 128, 4}, {512, 1, 512, 4},
     {64, 1, 64, 4}};
+
+// Size buckets of the tuning table, by pair count.  Below 2^25 pairs the chip
+// is short of workgroups and one-wave workgroups with many j-splits win by up
+// to 4 (split AccJerk 300 x 50000, pair kernel: 24 us, 108 at 512 x 2); above,
+// their one i per lane and short j ranges cost up to 1.25 (split AccJerk
+// 9000 x 7000: 89 us, 75 at two per lane; FP64 Acc 15000 x 15500: 196, 166).
+// From 2^30 the widest tiles are level or better.
+__host__ __device__ inline int size_bucket(int ni, int nj)
+{
+    const double pairs = static_cast<double>(ni) * static_cast<double>(nj);
+    if (pairs < 33554432.0) return 0;    // < 2^25
+    if (pairs < 1073741824.0) return 1;  // < 2^30
+    return 2;
+}
+
+// A shape whose workgroups would pad ni by more than a quarter (few i against
+// very many j) loses more than the one-wave shape of bucket 0 does.
+__host__ __device__ inline bool pads_rows(int ni, int block, int wpt)
+{
+    const long long rows = static_cast<long long>(block) * wpt;
+    return (ni + rows - 1) / rows * rows > ni + static_cast<long long>(ni) / 4;
+}
+
 // Below this many i-particles the j-split combine uses 8 lanes per i.
 constexpr int kWideReduceMaxNi = 32768;
 

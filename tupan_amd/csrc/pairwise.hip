@@ -357,14 +357,12 @@ static const int kPnShape[kShapes][4] = {
     {256, 1, 128, 1}, {128, 1, 128, 1}, {256, 1, 256, 2}, {64, 1, 64, 1}, {512, 1, 256, 1},
     {64, 1, 32, 1}};
 
-// Size buckets by pair count ni * nj.
-constexpr int kBuckets = 3;
-static int size_bucket(int ni, int nj)
+constexpr int kBuckets = kNumBuckets;
+static const int* shape_dims(int kernel, int shape)
 {
-    const double pairs = static_cast<double>(ni) * static_cast<double>(nj);
-    if (pairs < 4194304.0) return 0;        // < 2^22
-    if (pairs < 1073741824.0) return 1;     // < 2^30
-    return 2;
+    return kernel == K_SNAP_CRACKLE ? kHeavyShape[shape]
+           : kernel == K_PNACC      ? kPnShape[shape]
+                                    : kLightShape[shape];
 }
 
 // Tuning table: [kernel][mode slot][bucket] -> (shape, workgroups per CU).
@@ -389,9 +387,11 @@ static int launch_tuned(const Launcher<Op> (&table)[kShapes], int kernel, int sl
 {
     int rc = TUPAN_OK;
     if (run_sym<Op>(a, s, fixed, &rc)) return rc;
-    const TuneEntry& t = g_tune[kernel][slot][size_bucket(a.ni, a.nj)];
-    const int shape = (t.shape >= 0 && t.shape < kShapes) ? t.shape : 0;
-    return table[shape](a, s, t.wg_per_cu, fixed);
+    int b = size_bucket(a.ni, a.nj);
+    const int* d = shape_dims(kernel, g_tune[kernel][slot][b].shape);
+    if (pads_rows(a.ni, d[0], d[1])) b = 0;
+    const TuneEntry& t = g_tune[kernel][slot][b];
+    return table[t.shape](a, s, t.wg_per_cu, fixed);
 }
 
 #define TUPAN_RUN(Op, SHAPES, kernel, slot)                                      \
@@ -490,9 +490,7 @@ int tune_shape(int kernel, int shape, int* block, int* wpt, int* tile, int* unro
 {
     if (kernel < 0 || kernel >= kNumKernels || shape < 0 || shape >= kShapes)
         return set_error(TUPAN_ERR_ARG, "shape out of range");
-    const int* d = kernel == K_SNAP_CRACKLE ? kHeavyShape[shape]
-                   : kernel == K_PNACC      ? kPnShape[shape]
-                                            : kLightShape[shape];
+    const int* d = shape_dims(kernel, shape);
     if (block) *block = d[0];
     if (wpt) *wpt = d[1];
     if (tile) *tile = d[2];

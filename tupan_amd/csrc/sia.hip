@@ -787,7 +787,7 @@ struct LvlCtl {
     double bridge_c[kSubOps];
     int evolve_op[kSubOps];
     double evolve_c[kSubOps];
-    int tshape[2][3], twg[2][3];  // [0 Tstep, 1 Acc][size bucket]
+    int tshape[2][kNumBuckets], twg[2][kNumBuckets];  // [0 Tstep, 1 Acc][size bucket]
     double* partial;
     unsigned long long* tmp;  // narr x N, partition staging
     int* blk;                 // partition block counts, then offsets
@@ -799,14 +799,6 @@ namespace {
 __device__ __forceinline__ double* lvl_field(const LvlCtl* c, int role)
 {
     return reinterpret_cast<double*>(c->arr[c->role[role]]);
-}
-
-__device__ __forceinline__ int lvl_bucket(int ni, int nj)
-{
-    const double p = static_cast<double>(ni) * static_cast<double>(nj);
-    if (p < 4194304.0) return 0;
-    if (p < 1073741824.0) return 1;
-    return 2;
 }
 
 // The launch plan pairwise_call makes for Tstep (op 0) or Acc (op 1) of
@@ -871,7 +863,9 @@ __device__ void lvl_plan(LvlCtl* c, int op, int ilo, int ni, int jlo, int nj)
             return;
         }
     }
-    const int b = lvl_bucket(ni, nj);
+    int b = size_bucket(ni, nj);
+    if (pads_rows(ni, kLightShapeDims[c->tshape[op][b]][0], kLightShapeDims[c->tshape[op][b]][1]))
+        b = 0;
     const int shape = c->tshape[op][b];
     const int wg = c->twg[op][b];
     const int BLOCK = kLightShapeDims[shape][0], WPT = kLightShapeDims[shape][1],
@@ -1366,7 +1360,7 @@ int sia_levels_create(int n, void* const* arrays, int narrays, const int* roles,
         const int kernel = op == 0 ? K_TSTEP : K_ACC;
         const int mode = op == 0 ? tstep_mode : acc_mode;
         const int slot = mode == TUPAN_MODE_SPLIT32 ? 1 : 0;
-        for (int b = 0; b < 3; ++b) {
+        for (int b = 0; b < kNumBuckets; ++b) {
             int shape = 0, wg = 4;
             tune_get(kernel, slot, b, &shape, &wg);
             if (shape < 0 || shape >= kNumShapes) shape = 0;

@@ -1,10 +1,11 @@
 """Autotuner: ``python -m tupan_amd.tune [--quick]`` on the target GPU.
 
 For every pairwise kernel and arithmetic mode it times each compiled tile
-shape at 2, 4, 8 and 16 workgroups per CU on a uniform random cluster of one
-representative size per size bucket (1024, 16384 and 65536 particles, i =
-j), keeps the fastest (GPU time of the whole call, best of 3), and for the
-ensemble plan it times each lanes-per-system packing on the 4096-system
+shape at 2, 4, 8 and 16 workgroups per CU on calls between two random
+clusters of a few sizes per size bucket (few i against many j, square, many i
+against few j), and keeps the entry with the smallest mean of time over the
+best time of that size (GPU time of the whole call, combine included).  For
+the ensemble plan it times each lanes-per-system packing on the 4096-system
 workload.  The choices go to tupan_amd/tune/cache.json, which the library
 applies when it loads.
 """
@@ -20,18 +21,27 @@ from .. import _native
 from . import CACHE, load, save
 
 KERNELS = {  # name -> (kernel id, modes)
-    "phi": (_native.K_PHI, ("fp64",)),
-    "acc": (_native.K_ACC, ("fp64", "split32")),
-    "acc_jerk": (_native.K_ACC_JERK, ("fp64", "split32", "ieee64")),
-    "snap_crackle": (_native.K_SNAP_CRACKLE, ("fp64",)),
-    "tstep": (_native.K_TSTEP, ("fp64", "split32")),
-    "pnacc": (_native.K_PNACC, ("fp64", "split32")),
+    "phi": (_native.K_PHI, ("fp64", "float32")),
+    "acc": (_native.K_ACC, ("fp64", "split32", "float32")),
+    "acc_jerk": (_native.K_ACC_JERK, ("fp64", "split32", "ieee64",
+                                      "float32")),
+    "snap_crackle": (_native.K_SNAP_CRACKLE, ("fp64", "float32")),
+    "tstep": (_native.K_TSTEP, ("fp64", "split32", "float32")),
+    "nreg_x": (_native.K_NREG_X, ("fp64", "float32")),
+    "nreg_v": (_native.K_NREG_V, ("fp64", "float32")),
+    "pnacc": (_native.K_PNACC, ("fp64", "split32", "float32")),
 }
-SLOT = {"fp64": 0, "split32": 1, "ieee64": 2}
-BUCKET_N = (1024, 16384, 65536)
+# (ni, nj) of the calls timed per size bucket (below 2^25 pairs, below 2^30,
+# above)
+BUCKET_SETS = (
+    ((200, 3000), (64, 16000), (4000, 700), (2000, 2100), (300, 50000),
+     (16000, 700), (4000, 4096)),
+    ((2501, 60000), (9000, 7000), (15000, 15500), (60000, 2500), (30000, 31000)),
+    ((20000, 60000), (65000, 66000)),
+)
 
 
-def cluster(n, seed=0):
+def cluster(n, seed=0, dtype=torch.float64):
     from ..particles import ParticleSystem
     rng = np.random.default_rng(seed)
     d = {k: rng.normal(0, 1, n) for k in ("rx", "ry", "rz", "vx", "vy",
@@ -39,7 +49,31 @@ def cluster(n, seed=0):
                                          "jz")}
     d["mass"] = np.full(n, 1.0 / n)
     d["eps2"] = np.full(n, 1e-8)
-    return ParticleSystem.from_numpy(d, device="cuda:0")
+    ps = ParticleSystem.from_numpy(d, device="cuda:0")
+    if dtype != torch.float64:
+        for k, v in list(ps.arrays().items()):
+            if v.dtype == torch.float64:
+                ps.__dict__[k] = v.to(dtype)
+    return ps
+
+
+def queued_ms(fn, reps, hold):
+    """GPU time of one fn() in a run of `reps` behind a product of the
+    square matrix `hold`, which keeps the GPU busy while the host queues the
+    run: kernels and the gaps between them, no host time.  Best of 2."""
+    best = None
+    for _ in range(2):
+        t0 = torch.cuda.Event(enable_timing=True)
+        t1 = torch.cuda.Event(enable_timing=True)
+        torch.mm(hold, hold)
+        t0.record()
+        for _ in range(reps):
+            fn()
+        t1.record()
+        t1.synchronize()
+        t = t0.elapsed_time(t1) / reps
+        best = t if best is None else min(best, t)
+    return best
 
 
 def time_call(fn, reps):
@@ -62,47 +96,55 @@ def time_call(fn, reps):
 
 
 def tune_pairwise(quick, names):
+    from . import SLOTS
     from ..lib import extensions
     lib = _native.lib()
     out = []
-    sizes = BUCKET_N[:2] if quick else BUCKET_N
     # PNAcc at the reference's own test values (order 7, c = 128)
     extensions.clight.pn_order, extensions.clight.clight = 7, 128.0
-    for b, n in enumerate(sizes):
-        # the table serves calls between two sets (a set against itself
-        # above ~2000 particles takes the symmetric engine's own plan)
-        ps = cluster(n)
-        other = ps.copy()
+    hold = torch.ones(2048, 2048, dtype=torch.float64, device="cuda:0")
+    classes = {"phi": extensions.Phi, "acc": extensions.Acc,
+               "acc_jerk": extensions.AccJerk,
+               "snap_crackle": extensions.SnapCrackle,
+               "tstep": extensions.Tstep, "nreg_x": extensions.NREG_X,
+               "nreg_v": extensions.NREG_V, "pnacc": extensions.PNAcc}
+    for b, sets in enumerate(BUCKET_SETS[:2] if quick else BUCKET_SETS):
         for name, (kid, modes) in KERNELS.items():
             if name not in names:
                 continue
-            cls = {"phi": extensions.Phi, "acc": extensions.Acc,
-                   "acc_jerk": extensions.AccJerk,
-                   "snap_crackle": extensions.SnapCrackle,
-                   "tstep": extensions.Tstep,
-                   "pnacc": extensions.PNAcc}[name]
             for mode in modes:
-                ext = cls("HIP", "float64", mode=mode)
-                args = (0.01,) if name == "tstep" else ()
-                results = []
-                for shape in range(6):
-                    for wg in (2, 4, 8, 16):
-                        _native.check(lib.tupan_tune_set(kid, SLOT[mode], b,
-                                                         shape, wg),
-                                      "tupan_tune_set")
-                        t = time_call(lambda: ext.calc(ps, other, *args), 3)
-                        results.append((t, shape, wg))
-                results.sort()
-                t, shape, wg = results[0]
-                default = [r for r in results if r[1] == 0 and r[2] == 4][0]
-                _native.check(lib.tupan_tune_set(kid, SLOT[mode], b, shape,
+                flt = mode == "float32"
+                ext = (classes[name]("HIP", "float32") if flt else
+                       classes[name]("HIP", "float64", mode=mode))
+                args = (0.01,) if name in ("tstep", "nreg_x", "nreg_v") else ()
+                times = {}
+                for ni, nj in sets:
+                    dt = torch.float32 if flt else torch.float64
+                    ips, jps = cluster(ni, 0, dt), cluster(nj, 1, dt)
+                    reps = 10 if b == 0 else 2
+                    ext.calc(ips, jps, *args)
+                    for shape in range(6):
+                        for wg in (2, 4, 8, 16):
+                            _native.check(
+                                lib.tupan_tune_set(kid, SLOTS[mode], b, shape,
+                                                   wg), "tupan_tune_set")
+                            times.setdefault((shape, wg), []).append(queued_ms(
+                                lambda: ext.calc(ips, jps, *args), reps, hold))
+                best = [min(t[q] for t in times.values())
+                        for q in range(len(sets))]
+                score = {k: sum(x / y for x, y in zip(t, best)) / len(sets)
+                         for k, t in times.items()}
+                shape, wg = min(score, key=score.get)
+                _native.check(lib.tupan_tune_set(kid, SLOTS[mode], b, shape,
                                                  wg), "tupan_tune_set")
                 out.append({"kernel": name, "mode": mode, "bucket": b,
-                            "n": n, "shape": shape, "wg_per_cu": wg,
-                            "ms": t, "default_ms": default[0]})
-                print("%-12s %-7s n=%-6d shape %d wg/cu %d  %.3f ms "
-                      "(default %.3f)" % (name, mode, n, shape, wg, t,
-                                          default[0]), flush=True)
+                            "shape": shape, "wg_per_cu": wg,
+                            "over_best": round(score[shape, wg], 3),
+                            "default_over_best": round(score[0, 4], 3)})
+                print("%-12s %-7s bucket %d shape %d wg/cu %2d  %.3f x best "
+                      "(default %.3f)" % (name, mode, b, shape, wg,
+                                          score[shape, wg], score[0, 4]),
+                      flush=True)
     return out
 
 
