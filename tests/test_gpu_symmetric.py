@@ -88,6 +88,7 @@ CASES = ([(k, "fp64", n) for k in ("acc", "acc_jerk", "tstep", "snap_crackle")
           for n in FP64 if k == "acc_jerk" or n in (2049, 9217, 36865)]
          + [(k, "split32", n) for k in ("acc", "acc_jerk", "tstep")
             for n in FP32 if k == "acc_jerk" or n in (4097, 9217)]
+         + [("phi", "fp64", n) for n in (32768, 32769, 36865)]
          + [(k, "float", n) for k in CLASSES for n in (4097, 9217)])
 
 
@@ -109,7 +110,8 @@ def test_rows_vs_oracle(kernel, mode, n, soft):
             assert np.max(np.abs(g / r - 1)) <= bar
         return
     if kernel == "phi":
-        assert np.max(np.abs(got[0] / ref[0] - 1)) <= 2e-5
+        assert np.max(np.abs(got[0] / ref[0] - 1)) <= \
+            (1e-13 if mode == "fp64" else 2e-5)
         return
     if mode == "fp64":
         assert vec_rel_err(got[:3], ref[:3]) <= 1e-13

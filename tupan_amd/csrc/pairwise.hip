@@ -207,7 +207,7 @@ static bool run_sym(typename Op::Args a, hipStream_t stream, const FixedScratch*
 {
     if constexpr (kHasSym<Op>) {
         using S = typename SymOf<Op>::type;
-        if (a.exact || !same_set(a)) return false;
+        if (a.exact || a.ni <= kSymOpAbove<Op> || !same_set(a)) return false;
         const SymPlan p = sym_plan(a.ni, S::kK, sizeof(typename S::T) == 8,
                                    current_device().cu_count);
         if (p.shape < 0) return false;

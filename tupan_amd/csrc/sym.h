@@ -340,14 +340,12 @@ struct SymSplitTstep {
     __device__ static constexpr double scale() { return 1.0; }
 };
 
-// The policy of a tile-engine op, where there is one.  The FP64 Phi keeps the
-// tile engine, though a call takes 1.8 times as long there (n = 50000: 1.49
-// against 0.80 ms): initial conditions are drawn from it, and a seed's
-// realisation keeps its bits only with the potential's summation order.
+// The policy of a tile-engine op, where there is one.
 template <class Op>
 struct SymOf {
     using type = void;
 };
+template <> struct SymOf<OpPhi<Fast64>> { using type = SymPhi<Fast64>; };
 template <> struct SymOf<OpAcc<Fast64>> { using type = SymAcc<Fast64>; };
 template <> struct SymOf<OpAccJerk<Fast64>> { using type = SymAccJerk<Fast64>; };
 template <> struct SymOf<OpSnapCrackle<Fast64>> { using type = SymSnapCrackle<Fast64>; };
@@ -362,6 +360,16 @@ template <> struct SymOf<OpSplitAccJerk> { using type = SymSplitAccJerk; };
 template <> struct SymOf<OpSplitTstep> { using type = SymSplitTstep; };
 template <class Op>
 constexpr bool kHasSym = !std::is_void<typename SymOf<Op>::type>::value;
+// Largest set an op leaves to the tile engine whatever the plan below says.
+// Initial conditions are drawn from the FP64 Phi, and the 1e-14 comparison of
+// two pair solvers on the 16384-particle realisation depends on its last
+// bits, so a seed's realisation keeps the tile engine's summation order up to
+// 2^15 particles, where a potential costs under 0.7 ms (n = 32768: 0.67 there,
+// 0.40 here); beyond, the time counts (n = 50000: 1.49 against 0.87 ms).
+template <class Op>
+inline constexpr int kSymOpAbove = 0;
+template <>
+inline constexpr int kSymOpAbove<OpPhi<Fast64>> = 32768;
 
 // -- plan ---------------------------------------------------------------------
 // Shapes {W, TJ}: W particles per lane, TJ j-particles per LDS tile.

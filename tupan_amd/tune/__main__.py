@@ -95,7 +95,7 @@ def time_call(fn, reps):
     return best
 
 
-def tune_pairwise(quick, names):
+def tune_pairwise(quick, names, pinned=()):
     from . import SLOTS
     from ..lib import extensions
     lib = _native.lib()
@@ -113,6 +113,8 @@ def tune_pairwise(quick, names):
             if name not in names:
                 continue
             for mode in modes:
+                if (name, mode) in pinned:
+                    continue
                 flt = mode == "float32"
                 ext = (classes[name]("HIP", "float32") if flt else
                        classes[name]("HIP", "float64", mode=mode))
@@ -180,9 +182,13 @@ def main(argv=None):
     cu, _ = _native.device_info()
     t0 = time.time()
     old = load()
-    keep = [e for e in old.get("pairwise", []) if e.get("kernel") not in names]
+    # a pinned entry (FP64 phi: the summation order behind a seed's initial
+    # conditions) stays
+    keep = [e for e in old.get("pairwise", [])
+            if e.get("kernel") not in names or e.get("pinned")]
+    pinned = {(e["kernel"], e["mode"]) for e in keep if e.get("pinned")}
     data = {"device": {"cu": cu, "name": torch.cuda.get_device_name(0)},
-            "pairwise": keep + tune_pairwise(args.quick, names)}
+            "pairwise": keep + tune_pairwise(args.quick, names, pinned)}
     if args.ensemble_systems > 0:
         data["ensemble"] = tune_ensemble(args.ensemble_systems)
     elif "ensemble" in old:
