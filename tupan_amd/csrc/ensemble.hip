@@ -7,10 +7,10 @@
 // systems are sorted by size and each size bucket gets L lanes per system
 // (L in {8, 16, 32, 64}, at least the system size), so a wave holds 64/L
 // systems of similar size.  Lane l of a wave serves particle l % L of
-// system l / L and meets the others in rounds.  The lanes of a
-// wave step through their rounds together, so each lasts as long as
-// the slowest Kepler solve among the wave's pairs in it; grouping
-// systems of similar size keeps the lanes' round counts close.  Every lane
+// system l / L and meets the others in rounds.  The lanes of a wave step
+// through their rounds together, so each lasts as long as the slowest Kepler
+// solve among the wave's pairs in it; grouping systems of similar size keeps
+// the lanes' round counts close.  Every lane
 // stays in the wave to the end (inactive lanes compute nothing), so the
 // wave reductions of the work counters see all 64 lanes.
 //
@@ -24,8 +24,7 @@
 // The Sakura drift runs each plan wave as one workgroup of kEnsParts waves:
 // wave p takes the p-th of kEnsParts consecutive shares of the same lanes'
 // rounds (ensemble_sakura_body), and the partial sums are added in part order
-// (((d0 + d1) + d2) + d3), so a
-// launch has kEnsParts times as many, shorter waves to hide the solver's
+// (((d0 + d1) + d2) + d3), so a launch has kEnsParts times as many, shorter waves to hide the solver's
 // latency with (4 570 -> 12 416 waves for 4096 systems of U{3..64}).
 //
 // Compiled with -ffp-contract=off (reference operation order).
