@@ -49,11 +49,12 @@ PEAK_FP64 = 78.6e12          # MI355X vector FP64
 PEAK_FP32 = 157.3e12         # MI355X vector FP32 (counts packed FP32)
 HBM_PEAK = 8.0e12
 # HBM bytes per launch of the all-pairs kernel at N = 65536, from the two
-# calibrated rocprofv3 counter runs in profiles/accjerk_plummer65536_pmc_
-# traffic.md (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, KiB -> bytes).
+# rocprofv3 counter runs in profiles/symmetric_engine_counters.md, scaled as
+# profiles/accjerk_plummer65536_pmc_traffic.md calibrates the counters
+# (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, KiB -> bytes).
 TRAFFIC_65536 = {
-    "split32": (14871.8 * 2.0 + 196608.0) * 1024,
-    "fp64": (14637.1 * 2.0 + 98304.0) * 1024,
+    "split32": (84920.3 * 2.0 + 256512.0) * 1024,
+    "fp64": (50995.1 * 2.0 + 170496.0) * 1024,
 }
 
 
@@ -62,13 +63,14 @@ TRAFFIC_65536 = {
 # flop (sakura_kernel_common.h:45-123, 194-243: pair set-up and sums 36,
 # pre-drift 6, far/near test 13, leapfrog 32), and the hardware counts per
 # pair from rocprofv3 (SQ_INSTS_VALU x 64 / pairs, SQ_INSTS_VALU_FLOPS_FP64
-# x 64 / pairs; profiles/sakura_plummer16384_far_counters.md).
+# x 64 / pairs; profiles/symmetric_engine_counters.md): the kernel drifts each
+# unordered pair once, and the counts are per ordered pair of the call.
 SAKURA_FAR_REF_FLOPS = 87
-SAKURA_FAR_HW = {"valu_per_pair": 126.5, "fp64_flops_per_pair": 127.0}
+SAKURA_FAR_HW = {"valu_per_pair": 71.6, "fp64_flops_per_pair": 70.5}
 # Ensemble Sakura kernel (4096 systems, one pair-drift stage): hardware
 # counts per pair drift from the same profile (nearly every pair is a
 # Kepler solve, whose iterations the reference does not count).
-ENSEMBLE_HW = {"valu_per_pair": 2378.8, "fp64_flops_per_pair": 2097.2}
+ENSEMBLE_HW = {"valu_per_pair": 1360.2, "fp64_flops_per_pair": 1133.3}
 CLOCK_PEAK = 2.4e9           # MI355X peak engine clock
 SIMDS = 1024                 # 256 CUs x 4 SIMDs
 FP64_CYCLES_PER_WAVE_INSTR = 4
@@ -283,7 +285,7 @@ def sakura_roofline(pairs, far_s):
     hw = SAKURA_FAR_HW["fp64_flops_per_pair"] * pairs / far_s
     issue = SAKURA_FAR_HW["valu_per_pair"] * pairs / 64 / far_s
     peak_issue = SIMDS * CLOCK_PEAK / FP64_CYCLES_PER_WAVE_INSTR
-    return {"bound": "valu", "kernel": "sakura_far_kernel",
+    return {"bound": "valu", "kernel": "sakura_far_sym_kernel",
             "achieved": alg / 1e12, "peak": PEAK_FP64 / 1e12,
             "unit": "TFLOP/s", "frac": alg / PEAK_FP64,
             "flops_per_pair": SAKURA_FAR_REF_FLOPS,
@@ -997,8 +999,9 @@ def main():
         "bound_note": "vector-ALU compute: the pair interaction is not a "
                       "contraction, so no MFMA; peak is the published FP32 "
                       "vector peak, achieved counts the reference's 42 flops "
-                      "per pair",
-        "kernel": "pair_kernel<OpSplitAccJerk>",
+                      "per ordered pair (the kernel evaluates each "
+                      "unordered pair once)",
+        "kernel": "sym_kernel<SymSplitAccJerk>",
         "achieved": flops / k_split / 1e12,
         "peak": PEAK_FP32 / 1e12,
         "unit": "TFLOP/s",
@@ -1006,7 +1009,7 @@ def main():
         "traffic": TRAFFIC_65536["split32"] if n == 65536 else None,
         "traffic_unit": "bytes per launch (rocprofv3 FETCH_SIZE, WRITE_SIZE)",
         "algorithmic_bytes": (8 + 6) * 8 * n,
-        "fp64_kernel": {"kernel": "pair_kernel<OpAccJerk<Fast64>>",
+        "fp64_kernel": {"kernel": "sym_kernel<SymAccJerk<Fast64>>",
                         "achieved": flops / k_fp64 / 1e12,
                         "peak": PEAK_FP64 / 1e12,
                         "frac": flops / k_fp64 / PEAK_FP64},
