@@ -97,3 +97,25 @@ def test_other_arrays_keep_the_array_operations():
          for _ in range(6)]
     assert not device_update(DRIFT, y, 0.5)
     assert not device_update(DRIFT, [t.cpu() for t in y], 0.5)
+
+
+@pytest.mark.parametrize("narr", [1, 3, 4, 5, 16, 31, 32])
+@pytest.mark.parametrize("n", [7, 1025])
+def test_partition_moves_every_array(n, narr):
+    """Array counts around the four that a block moves, the first array the
+    step sizes themselves: order and bits of a stable partition."""
+    import ctypes as C
+    from tupan_amd import _native
+    g = torch.Generator(device="cuda:0").manual_seed(n + narr)
+    arrs = [torch.rand(n, dtype=torch.float64, device="cuda:0", generator=g)
+            for _ in range(narr)]
+    slow = arrs[0] > 0.4
+    ref = [torch.cat((a[slow], a[~slow])) for a in arrs]
+    ptrs = (C.c_void_p * narr)(*[a.data_ptr() for a in arrs])
+    out = (C.c_int * 2)()
+    _native.check(_native.lib().tupan_sia_split(
+        n, ptrs, narr, arrs[0].data_ptr(), 0.4, None, out,
+        torch.cuda.current_stream().cuda_stream), "tupan_sia_split")
+    assert out[0] == int(slow.sum()) and out[1] == 0
+    for a, r in zip(arrs, ref):
+        assert torch.equal(a, r)
