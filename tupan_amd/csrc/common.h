@@ -49,8 +49,17 @@ __device__ __forceinline__ double rsqrt_refined(double x)
 // waves per SIMD, 3.7 cycles per instruction without and 2.35 with (2.3
 // with no v_rsq_f32 at all).  The s_nop is the wait state a plain VALU
 // consumer of the result needs.
+//
+// Not for kernels with at most about one wave per SIMD (kRaise false): alone
+// on its SIMD a wave only pays the three extra instructions (split Tstep
+// 1000 x 2000: 9.7 us without, 10.4 with), and a load moved behind the asm
+// block is no longer merged with its neighbours: the small-set kernel's
+// 16-byte LDS reads became 4-byte ones with bank conflicts (float
+// SnapCrackle, n = 1400: 12.4 -> 39.7 us).
+template <bool kRaise = true>
 __device__ __forceinline__ float rsq_f32(float x)
 {
+    if constexpr (!kRaise) return __builtin_amdgcn_rsqf(x);
     float y;
     asm("s_setprio 3\n\tv_rsq_f32 %0, %1\n\ts_nop 0\n\ts_setprio 0" : "=v"(y) : "v"(x));
     return y;
@@ -58,9 +67,10 @@ __device__ __forceinline__ float rsq_f32(float x)
 
 // FP32: v_rsq_f32 refined by one first-order Newton step (the estimate is
 // already within about one ulp; the step removes its bias).
+template <bool kRaise = true>
 __device__ __forceinline__ float rsqrt_refined(float x)
 {
-    float y0 = rsq_f32(x);
+    float y0 = rsq_f32<kRaise>(x);
     float h = x * y0;
     float e = __builtin_fmaf(-h, y0, 1.0f);
     return __builtin_fmaf(0.5f * y0, e, y0);

@@ -253,7 +253,7 @@ struct OpAccJerkTstep {
     using Args = PairArgs<double>;
     using Frame = typename AJ::Frame;
     using Slot = typename AJ::Slot;
-    static constexpr bool kSplit = std::is_same<AJ, OpSplitAccJerk>::value;
+    static constexpr bool kSplit = std::is_same<AJ, Lone<OpSplitAccJerk>>::value;
     static_assert(std::is_same<Slot, typename TS::Slot>::value,
                   "one slot layout serves both interactions");
     struct IReg { typename AJ::IReg a; typename TS::IReg t; };
@@ -461,7 +461,8 @@ int step_order(int adaptive, int mode, int n, const HermiteArrays& h, double eta
     if constexpr (Order == 4) {
         if (adaptive && fused4(mode, n)) {
             return mode == TUPAN_MODE_SPLIT32
-                       ? fused_adaptive_step4<OpSplitAccJerk, OpSplitTstep>(n, h, eta, ctl, s)
+                       ? fused_adaptive_step4<Lone<OpSplitAccJerk>, Lone<OpSplitTstep>>(n, h, eta,
+                                                                                    ctl, s)
                        : fused_adaptive_step4<OpAccJerk<Fast64>, OpTstep<Fast64>>(n, h, eta,
                                                                                   ctl, s);
         }
@@ -479,7 +480,7 @@ int step_order(int adaptive, int mode, int n, const HermiteArrays& h, double eta
     if constexpr (Order == 4) {
         if (fused4(mode, n)) {
             return mode == TUPAN_MODE_SPLIT32
-                       ? fused_step4<OpSplitAccJerk>(n, h, ctl, adaptive, s)
+                       ? fused_step4<Lone<OpSplitAccJerk>>(n, h, ctl, adaptive, s)
                        : fused_step4<OpAccJerk<Fast64>>(n, h, ctl, adaptive, s);
         }
     }

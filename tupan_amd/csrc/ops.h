@@ -50,21 +50,24 @@ struct Fast64 {
     }
 };
 
-struct Fast32 {
+// kRaise: common.h, rsq_f32.
+template <bool kRaise>
+struct Fast32T {
     using T = float;
     static constexpr bool kFused = true;
     __device__ static __forceinline__ void q12(T r2, T e2, bool mask, T& q1, T& q2)
     {
-        T y = rsqrt_refined(r2 + e2);
+        T y = rsqrt_refined<kRaise>(r2 + e2);
         y = mask ? y : T(0);
         q1 = y;
         q2 = y * y;
     }
     __device__ static __forceinline__ T eta_over_sqrt(T eta, T w2)
     {
-        return eta * rsqrt_refined(w2);
+        return eta * rsqrt_refined<kRaise>(w2);
     }
 };
+using Fast32 = Fast32T<true>;
 
 struct Ieee64 {
     using T = double;
@@ -596,11 +599,11 @@ constexpr double kRsqBias = -7.35832e-9;
 
 // kMask false: no R^2 > e2 test (the unmasked tiles of the split Acc and
 // AccJerk, see their self_safe).
-template <bool kRefine, bool kMask = true>
+template <bool kRefine, bool kMask = true, bool kRaise = true>
 __device__ __forceinline__ float split_rsqrt(float dx, float dy, float dz, float e2)
 {
     const float R2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, e2)));
-    const float y = kRefine ? rsqrt_refined(R2) : rsq_f32(R2);
+    const float y = kRefine ? rsqrt_refined<kRaise>(R2) : rsq_f32<kRaise>(R2);
     if constexpr (!kMask) return y;
     return R2 > e2 ? y : 0.0f;
 }
@@ -619,7 +622,7 @@ constexpr double split_scale()
     return kRefine ? 1.0 : 1.0 / (1.0 + 3.0 * kRsqBias);
 }
 
-template <bool kRefine>
+template <bool kRefine, bool kRaise = true>
 struct OpSplitAccT {
     using Args = PairArgs<double>;
     using Frame = SplitFrame;
@@ -689,7 +692,7 @@ struct OpSplitAccT {
         float dy = (r.yh - s.v[1]) + (r.yl - s.v[5]);
         float dz = (r.zh - s.v[2]) + (r.zl - s.v[6]);
         const float y =
-            split_rsqrt<kRefine, kM || !kU>(dx, dy, dz, kU ? e2u : r.e2 + s.v[7]);
+            split_rsqrt<kRefine, kM || !kU, kRaise>(dx, dy, dz, kU ? e2u : r.e2 + s.v[7]);
         float q3 = (y * y) * (y * s.v[3]);
         c.ax = __builtin_fmaf(-q3, dx, c.ax);
         c.ay = __builtin_fmaf(-q3, dy, c.ay);
@@ -715,7 +718,7 @@ struct OpSplitAccT {
     }
 };
 
-template <bool kRefine>
+template <bool kRefine, bool kRaise = true>
 struct OpSplitAccJerkT {
     using Args = PairArgs<double>;
     using Frame = SplitFrame;
@@ -803,7 +806,7 @@ struct OpSplitAccJerkT {
         float uy = r.vy - s.v[9];
         float uz = r.vz - s.v[10];
         float rv = __builtin_fmaf(dz, uz, __builtin_fmaf(dy, uy, dx * ux));
-        const float y = split_rsqrt<kRefine, kM || !kU>(dx, dy, dz, e2);
+        const float y = split_rsqrt<kRefine, kM || !kU, kRaise>(dx, dy, dz, e2);
         float q2 = y * y;
         float q3 = q2 * (y * s.v[3]);
         float alpha = 3.0f * rv * q2;
@@ -846,7 +849,8 @@ struct OpSplitAccJerkT {
 // total masses near 1 (a softening of 1e-4 keeps every R above it); an i
 // whose FP32 sums overflow there is evaluated again by OpTstep<Fast64>
 // (engine.h: fallback64).
-struct OpSplitTstep {
+template <bool kRaise>
+struct OpSplitTstepT {
     using Args = PairArgs<double>;
     using Frame = SplitFrame;
     using Fallback64 = OpTstep<Fast64>;
@@ -910,12 +914,12 @@ struct OpSplitTstep {
         float v2 = __builtin_fmaf(uz, uz, __builtin_fmaf(uy, uy, ux * ux));
         const bool mask = R2 > e2;
         // no mask on 1/R: a masked pair's term is zeroed at the end
-        float q1 = rsq_f32(R2);
+        float q1 = rsq_f32<kRaise>(R2);
         float q2 = q1 * q1;
         float phi2 = mt * q1;  // 2 phi: mt is the doubled mass sum
         float w2 = q2 * (phi2 + v2);
         float ga = q2 * __builtin_fmaf(q2, phi2, w2);
-        ga *= r.eta * rsq_f32(w2);
+        ga *= r.eta * rsq_f32<kRaise>(w2);
         w2 = __builtin_fmaf(-ga, rv, w2);
         return mask ? w2 : 0.0f;
     }
@@ -1099,5 +1103,31 @@ struct OpNregV {
 constexpr bool kSplitRefine = TUPAN_SPLIT_REFINE != 0;
 using OpSplitAcc = OpSplitAccT<kSplitRefine>;
 using OpSplitAccJerk = OpSplitAccJerkT<kSplitRefine>;
+using OpSplitTstep = OpSplitTstepT<true>;
+
+// The op for kernels that leave about one wave per SIMD: the same arithmetic
+// with FP32 reciprocal roots at the wave's own priority (common.h, rsq_f32).
+template <class Op>
+struct LoneOf {
+    using type = Op;
+};
+template <template <class> class O>
+struct LoneOf<O<Fast32>> {
+    using type = O<Fast32T<false>>;
+};
+template <bool R>
+struct LoneOf<OpSplitAccT<R, true>> {
+    using type = OpSplitAccT<R, false>;
+};
+template <bool R>
+struct LoneOf<OpSplitAccJerkT<R, true>> {
+    using type = OpSplitAccJerkT<R, false>;
+};
+template <>
+struct LoneOf<OpSplitTstepT<true>> {
+    using type = OpSplitTstepT<false>;
+};
+template <class Op>
+using Lone = typename LoneOf<Op>::type;
 
 }  // namespace tupan

@@ -256,7 +256,7 @@ static int run_pairwise(typename Op::Args a, hipStream_t stream, int wg_per_cu,
         constexpr int ipb = kSmallBlock / kSmallGroups;
         const unsigned grid = static_cast<unsigned>((a.ni + ipb - 1) / ipb);
         if (!fixed) timing_begin(stream);
-        hipLaunchKernelGGL((pair_small_kernel<Op, kSmallBlock, kSmallGroups, small_tile<Op>()>),
+        hipLaunchKernelGGL((pair_small_kernel<Lone<Op>, kSmallBlock, kSmallGroups, small_tile<Op>()>),
                            dim3(grid), dim3(kSmallBlock), 0, stream, a);
         if (!fixed) timing_end(stream);
         launch_post_fallback<Op>(a, stream);
@@ -302,8 +302,17 @@ static int run_pairwise(typename Op::Args a, hipStream_t stream, int wg_per_cu,
     }
     const unsigned grid = static_cast<unsigned>(L.nblock_i) * static_cast<unsigned>(L.nsplit);
     if (!fixed) timing_begin(stream);
-    hipLaunchKernelGGL((pair_kernel<Op, BLOCK, WPT, TILE, UNROLL>), dim3(grid), dim3(BLOCK), 0,
-                       stream, a);
+    // at most a wave to a SIMD: no raised priority
+    bool lone = false;
+    if constexpr (BLOCK == kWave) {
+        lone = grid <= 4u * static_cast<unsigned>(dev.cu_count);
+        if (lone)
+            hipLaunchKernelGGL((pair_kernel<Lone<Op>, BLOCK, WPT, TILE, UNROLL>), dim3(grid),
+                               dim3(BLOCK), 0, stream, a);
+    }
+    if (!lone)
+        hipLaunchKernelGGL((pair_kernel<Op, BLOCK, WPT, TILE, UNROLL>), dim3(grid), dim3(BLOCK), 0,
+                           stream, a);
     if (!fixed) timing_end(stream);
     if (L.nsplit > 1) {
         if (a.ni <= kWideReduceMaxNi) {

@@ -125,7 +125,7 @@ __device__ void pair_op(const SubtreeArgs& a, int ilo, int ni, int jlo, int nj, 
 __device__ void acc_op(const SubtreeArgs& a, int ilo, int ni, int jlo, int nj)
 {
     if (a.acc_mode == TUPAN_MODE_SPLIT32) {
-        pair_op<OpSplitAcc>(a, ilo, ni, jlo, nj, 0.0, field(a, R_AX), field(a, R_AY),
+        pair_op<Lone<OpSplitAcc>>(a, ilo, ni, jlo, nj, 0.0, field(a, R_AX), field(a, R_AY),
                             field(a, R_AZ));
     } else {
         pair_op<OpAcc<Fast64>>(a, ilo, ni, jlo, nj, 0.0, field(a, R_AX), field(a, R_AY),
@@ -137,7 +137,7 @@ __device__ void acc_op(const SubtreeArgs& a, int ilo, int ni, int jlo, int nj)
 __device__ void tstep_op(const SubtreeArgs& a, int lo, int n)
 {
     if (a.tstep_mode == TUPAN_MODE_SPLIT32) {
-        pair_op<OpSplitTstep>(a, lo, n, lo, n, a.eta, field(a, R_TSTEP), field(a, R_TSTEPIJ),
+        pair_op<Lone<OpSplitTstep>>(a, lo, n, lo, n, a.eta, field(a, R_TSTEP), field(a, R_TSTEPIJ),
                               nullptr);
     } else {
         pair_op<OpTstep<Fast64>>(a, lo, n, lo, n, a.eta, field(a, R_TSTEP),
@@ -1087,7 +1087,7 @@ __global__ __launch_bounds__(kSmallBlock) void lvl_small_kernel(const LvlCtl* c,
     if (c->kind != LK_PAIR || c->op != op || c->cand != kCandSmall) return;
     const int bid = static_cast<int>(blockIdx.x);
     if (bid >= c->grid) return;
-    pair_small_body<Op, kSmallBlock, kSmallGroups, small_tile<Op>()>(c->pa, bid);
+    pair_small_body<Lone<Op>, kSmallBlock, kSmallGroups, small_tile<Op>()>(c->pa, bid);
 }
 
 template <class Op, int S>
