@@ -737,13 +737,18 @@ int sia_update_call(int kind, size_t n, void* const* arrays, double h, void* str
 // sia_subtree_kernel.  Here the same walk is a state machine in device
 // memory (LvlCtl: a stack of level frames and a queue of pending
 // operations), advanced by lvl_sched_kernel, one operation per "slot".  A
-// slot is the scheduler followed by one launch of every worker kernel: the
-// tile engine in each tile shape the tuning table uses for Tstep and Acc,
-// the small-set kernel and both split combines, the four partition passes,
-// the elementwise updates, the subtree kernel and the few-body kernel.  Each
-// worker reads the descriptor the scheduler wrote and exits unless the slot
-// is its own, so the launch sequence is fixed and a run of slots can be
-// captured as one HIP graph and replayed until the step's stack is empty.
+// slot is the scheduler followed by one launch of every worker kernel: for
+// Tstep and Acc the tile engine and the symmetric engine in the shapes that
+// calls of a set of N can take (lvl_workers), the small-set kernel and the
+// combines, the four partition passes, the elementwise updates, the subtree
+// kernel and the few-body kernel.  Each worker reads the descriptor the
+// scheduler wrote and exits unless the slot is its own, so the launch
+// sequence is fixed and a run of slots can be captured as one HIP graph and
+// replayed until the step's stack is empty.  A slot costs its launches, most
+// of them empty (about 2 us each, more with thousands of workgroups): a
+// worker no call can reach is not launched, and grids are no larger than the
+// largest plan (sia21h step, FP64, N = 3000: 464 ms with every shape of the
+// table at its target's grid, 288 ms; N = 12000: 1055 and 760 ms).
 //
 // Every operation is the host driver's, in its order, with its launch plan:
 // the scheduler plans each Tstep and Acc call exactly as pairwise_call does
@@ -763,6 +768,7 @@ constexpr int kLvlVisits = 1 << 20;  // level visits per step
 constexpr int kPartPer = 1024;       // particles per partition block (256 x 4)
 constexpr int kCandSmall = kNumShapes;  // candidate id of the small-set kernel
 constexpr int kCandSym = kNumShapes + 1;  // of the symmetric engine's first shape
+constexpr int kNumCands = kCandSym + kNumSymShapes;
 
 enum { LK_NONE = 0, LK_PAIR = 1, LK_PART = 2, LK_ELEM = 3, LK_SUBTREE = 4, LK_FEW = 5 };
 enum { MT_TSTEP, MT_ACC, MT_PART, MT_DRIFT, MT_KICK, MT_FEW, MT_PUSH };
@@ -804,6 +810,8 @@ struct LvlCtl {
     int evolve_op[kSubOps];
     double evolve_c[kSubOps];
     int tshape[2][kNumBuckets], twg[2][kNumBuckets];  // [0 Tstep, 1 Acc][size bucket]
+    // grids of the workers in a slot, 0: none (candidate ids as `cand`)
+    int gmax[2][kNumCands];
     double* partial;
     unsigned long long* tmp;  // narr x N, partition staging
     int* blk;                 // partition block counts, then offsets
@@ -819,9 +827,8 @@ __device__ __forceinline__ double* lvl_field(const LvlCtl* c, int role)
 
 // The launch plan pairwise_call makes for Tstep (op 0) or Acc (op 1) of
 // i in [ilo, ilo + ni) against j in [jlo, jlo + nj), written to the
-// descriptor.  Returns false if the planned shape has no worker in the
-// slots (the tuning table changed since the slots were enqueued).
-__device__ void lvl_plan(LvlCtl* c, int op, int ilo, int ni, int jlo, int nj)
+// descriptor.
+__device__ void lvl_plan_pair(LvlCtl* c, int op, int ilo, int ni, int jlo, int nj)
 {
     PairArgs<double>& a = c->pa;
     const int fr[8] = {R_MASS, R_RX, R_RY, R_RZ, R_E2, R_VX, R_VY, R_VZ};
@@ -903,6 +910,17 @@ __device__ void lvl_plan(LvlCtl* c, int op, int ilo, int ni, int jlo, int nj)
             c->comb = 2;
             c->comb_grid = (ni + 255) / 256;
         }
+    }
+}
+
+// The same, and status bit 8 if the slots hold no worker for the plan.
+__device__ void lvl_plan(LvlCtl* c, int op, int ilo, int ni, int jlo, int nj)
+{
+    lvl_plan_pair(c, op, ilo, ni, jlo, nj);
+    if (c->grid > c->gmax[op][c->cand] || (c->comb == 2 && c->N <= kWideReduceMaxNi)) {
+        c->kind = LK_NONE;
+        c->status |= kLvlErrPlan;
+        c->done = 1;
     }
 }
 
@@ -1100,27 +1118,36 @@ __global__ __launch_bounds__(kSymBlock) void lvl_sym_kernel(const LvlCtl* c, int
                                                                                  c->sym_nb);
 }
 
-template <class Op>
-__global__ __launch_bounds__(kSymReduceWaves* kWave) void lvl_sym_reduce_kernel(const LvlCtl* c,
-                                                                                int op)
+// The combines serve Tstep (OpT) and Acc (OpA) from one launch.
+template <class OpT, class OpA>
+__global__ __launch_bounds__(kSymReduceWaves* kWave) void lvl_sym_reduce_kernel(const LvlCtl* c)
 {
-    if (c->kind != LK_PAIR || c->op != op || c->comb != 3) return;
+    if (c->kind != LK_PAIR || c->comb != 3) return;
     const int bid = static_cast<int>(blockIdx.x);
     if (bid >= c->comb_grid) return;
-    sym_reduce_body<typename SymOf<Op>::type>(
-        c->pa, bid, c->sym_nb, kSymBlock * kSymShapeDims[c->cand - kCandSym][0]);
+    const int bi = kSymBlock * kSymShapeDims[c->cand - kCandSym][0];
+    if (c->op == 0)
+        sym_reduce_body<typename SymOf<OpT>::type>(c->pa, bid, c->sym_nb, bi);
+    else
+        sym_reduce_body<typename SymOf<OpA>::type>(c->pa, bid, c->sym_nb, bi);
 }
 
-template <class Op>
-__global__ __launch_bounds__(256) void lvl_combine_kernel(const LvlCtl* c, int op, int wide)
+template <class OpT, class OpA, bool kWide>
+__global__ __launch_bounds__(256) void lvl_combine_kernel(const LvlCtl* c)
 {
-    if (c->kind != LK_PAIR || c->op != op || c->comb != (wide ? 1 : 2)) return;
+    if (c->kind != LK_PAIR || c->comb != (kWide ? 1 : 2)) return;
     const int bid = static_cast<int>(blockIdx.x);
     if (bid >= c->comb_grid) return;
-    if (wide) {
-        reduce_wide_body<Op, 8>(c->pa, bid);
+    if constexpr (kWide) {
+        if (c->op == 0)
+            reduce_wide_body<OpT, 8>(c->pa, bid);
+        else
+            reduce_wide_body<OpA, 8>(c->pa, bid);
     } else {
-        reduce_body<Op>(c->pa, bid);
+        if (c->op == 0)
+            reduce_body<OpT>(c->pa, bid);
+        else
+            reduce_body<OpA>(c->pa, bid);
     }
 }
 
@@ -1318,10 +1345,73 @@ struct LevelsPlan {
     int* blk = nullptr;
     int N = 0;
     int tstep_mode = 0, acc_mode = 0;
-    int shapes[2][kNumShapes] = {};   // shapes the tuning table uses, per op
-    int grid_max[2][kNumShapes] = {};
-    int sym_grid[2][kNumSymShapes] = {};  // largest grids of the symmetric engine, 0: unused
+    int gmax[2][kNumCands] = {};  // worker grids per op and candidate, 0: not launched
 };
+
+namespace {
+
+// The workers that Tstep and Acc calls of a set of n can reach, their largest
+// grids (h.gmax), and the partial sums (doubles) of the largest plan.  Tstep
+// calls are a level's set against itself, Acc calls also its two parts
+// against each other.
+size_t lvl_workers(LvlCtl& h, int n)
+{
+    size_t part = 0;
+    const int top = n / 2, rest = n - top;
+    for (int op = 0; op < 2; ++op) {
+        const int nacc = op == 0 ? 2 : 3;
+        const bool fp64 = (op == 0 ? h.tstep_mode : h.acc_mode) != TUPAN_MODE_SPLIT32;
+        int last_bucket = op == 0 ? 0 : size_bucket(top, rest);
+        // a set against itself is at most 2^24 pairs where the symmetric
+        // engine does not take it, unless its partial sums are over the limit
+        static_assert(kSymAbove64 <= 4096 && kSymAbove32 <= 4096, "bucket 0 below the engine");
+        // the symmetric engine: a plan's counts depend on the size through
+        // its block count, so the multiples of the smallest block and n
+        // cover every size
+        for (long long q = kSymBlock;; q += kSymBlock) {
+            const int m = static_cast<int>(q < n ? q : n);
+            if (sym_shape(m, fp64) >= 0) {
+                const SymPlan sp = sym_plan(m, nacc, fp64, h.cu_count);
+                if (sp.shape < 0) {
+                    const int b = size_bucket(n, n);
+                    if (b > last_bucket) last_bucket = b;
+                } else {
+                    int& g = h.gmax[op][kCandSym + sp.shape];
+                    if (sp.nb * sp.nchunk > g) g = sp.nb * sp.nchunk;
+                    const size_t need = sym_doubles(sp, nacc, m);
+                    if (need > part) part = need;
+                }
+            }
+            if (m == n) break;
+        }
+        const int small_ipb = kSmallBlock / kSmallGroups;
+        // nj > kSmallMinJ, so ni <= kSmallPairs / kSmallMinJ
+        const long long small_ni =
+            n < kSmallPairs / kSmallMinJ ? n : kSmallPairs / kSmallMinJ;
+        h.gmax[op][kCandSmall] = static_cast<int>((small_ni + small_ipb - 1) / small_ipb);
+        for (int b = 0; b <= last_bucket; ++b) {
+            const int s = h.tshape[op][b];
+            const int ipb = kLightShapeDims[s][0] * kLightShapeDims[s][1];
+            const int wg = h.twg[op][b] > 0 ? h.twg[op][b] : 4;
+            const long long target = static_cast<long long>(wg) * h.cu_count;
+            const long long nblk = (n + ipb - 1) / ipb;
+            // plan_launch: nblock_i * nsplit is at most target + nblock_i, or
+            // twice a count below 8 per CU, plus nblock_i; no split has fewer
+            // than 32 j
+            const long long few = 16ll * h.cu_count;
+            long long g = (target > few ? target : few) + nblk + 1;
+            const long long cut = nblk * ((n + 31) / 32);
+            if (cut < g) g = cut;
+            int& have = h.gmax[op][s];
+            if (g > have) have = static_cast<int>(g);
+            const size_t need = static_cast<size_t>(nacc) * static_cast<size_t>(g) * ipb;
+            if (need > part) part = need;
+        }
+    }
+    return part;
+}
+
+}  // namespace
 
 int sia_levels_create(int n, void* const* arrays, int narrays, const int* roles, int acc_mode,
                       int tstep_mode, double eta, int nbridge, const int* bridge_op,
@@ -1369,9 +1459,7 @@ int sia_levels_create(int n, void* const* arrays, int narrays, const int* roles,
     p->N = n;
     p->tstep_mode = tstep_mode;
     p->acc_mode = acc_mode;
-    // the tuning table's shapes for Tstep and Acc in these modes, and each
-    // shape's largest grid over calls of at most n x n pairs
-    int wg_max[2][kNumShapes] = {};
+    // the tuning table's shapes for Tstep and Acc in these modes
     for (int op = 0; op < 2; ++op) {
         const int kernel = op == 0 ? K_TSTEP : K_ACC;
         const int mode = op == 0 ? tstep_mode : acc_mode;
@@ -1382,47 +1470,11 @@ int sia_levels_create(int n, void* const* arrays, int narrays, const int* roles,
             if (shape < 0 || shape >= kNumShapes) shape = 0;
             h.tshape[op][b] = shape;
             h.twg[op][b] = wg;
-            p->shapes[op][shape] = 1;
-            const int w = wg > 0 ? wg : 4;
-            if (w > wg_max[op][shape]) wg_max[op][shape] = w;
         }
     }
-    size_t part_doubles = 0;
-    for (int op = 0; op < 2; ++op) {
-        const size_t nacc = op == 0 ? 2 : 3;
-        for (int s = 0; s < kNumShapes; ++s) {
-            if (!p->shapes[op][s]) continue;
-            const int ipb = kLightShapeDims[s][0] * kLightShapeDims[s][1];
-            const long long target = static_cast<long long>(wg_max[op][s]) * h.cu_count;
-            const long long nblk = (n + ipb - 1) / ipb;
-            // plan_launch: nblock_i * nsplit is at most target + nblock_i, or
-            // twice a count below 8 per CU, plus nblock_i
-            const long long few = 16ll * h.cu_count;
-            p->grid_max[op][s] = static_cast<int>((target > few ? target : few) + nblk + 1);
-            const size_t need = nacc * static_cast<size_t>(p->grid_max[op][s]) * ipb;
-            if (need > part_doubles) part_doubles = need;
-        }
-    }
-    // the symmetric engine's largest grid per shape and its partial sums over
-    // every set size: a plan's counts depend on the size through its block
-    // count, so the multiples of the smallest block and n cover them
-    for (int op = 0; op < 2; ++op) {
-        const int nacc = op == 0 ? 2 : 3;
-        const bool fp64 = (op == 0 ? tstep_mode : acc_mode) != TUPAN_MODE_SPLIT32;
-        for (long long q = kSymBlock;; q += kSymBlock) {
-            const int m = static_cast<int>(q < n ? q : n);
-            const int shape = sym_shape(m, fp64);
-            if (shape >= 0) {
-                const SymPlan sp = sym_plan(m, nacc, fp64, h.cu_count);
-                const int grid = sp.nb * sp.nchunk;
-                if (grid > p->sym_grid[op][shape]) p->sym_grid[op][shape] = grid;
-                size_t need = sym_doubles(sp, nacc, m);
-                if (need > kSymMaxBytes / sizeof(double)) need = kSymMaxBytes / sizeof(double);
-                if (need > part_doubles) part_doubles = need;
-            }
-            if (m == n) break;
-        }
-    }
+    const size_t part_doubles = lvl_workers(h, n);
+    for (int op = 0; op < 2; ++op)
+        for (int k = 0; k < kNumCands; ++k) p->gmax[op][k] = h.gmax[op][k];
     const size_t nb = (static_cast<size_t>(n) + kPartPer - 1) / kPartPer;
     int rc = check_hip(hipMalloc(&p->ctl, sizeof(LvlCtl)), "levels control");
     if (rc == TUPAN_OK)
@@ -1466,14 +1518,13 @@ int sia_levels_destroy(void* plan)
 namespace {
 
 template <class Op>
-int lvl_enqueue_pair_workers(const LevelsPlan* p, int op, hipStream_t s)
+void lvl_enqueue_op(const LevelsPlan* p, int op, hipStream_t s)
 {
-    // one launch per shape the tuning table uses, the small-set kernel, the
-    // two combines, the symmetric engine's shapes and its reduction
-#define TUPAN_LVL_SHAPE(S)                                                                   \
-    if (p->shapes[op][S])                                                                    \
-        hipLaunchKernelGGL((lvl_pair_kernel<Op, S>), dim3(p->grid_max[op][S]),               \
-                           dim3(kLightShapeDims[S][0]), 0, s, p->ctl, op);
+    const int* g = p->gmax[op];
+#define TUPAN_LVL_SHAPE(S)                                                              \
+    if (g[S])                                                                           \
+        hipLaunchKernelGGL((lvl_pair_kernel<Op, S>), dim3(g[S]), dim3(kLightShapeDims[S][0]), \
+                           0, s, p->ctl, op);
     TUPAN_LVL_SHAPE(0)
     TUPAN_LVL_SHAPE(1)
     TUPAN_LVL_SHAPE(2)
@@ -1481,26 +1532,35 @@ int lvl_enqueue_pair_workers(const LevelsPlan* p, int op, hipStream_t s)
     TUPAN_LVL_SHAPE(4)
     TUPAN_LVL_SHAPE(5)
 #undef TUPAN_LVL_SHAPE
-    constexpr int ipb = kSmallBlock / kSmallGroups;
-    // the small-set path has nj > kSmallMinJ, so ni <= kSmallPairs / kSmallMinJ
-    const int small_grid = static_cast<int>((kSmallPairs / kSmallMinJ + ipb - 1) / ipb);
-    hipLaunchKernelGGL((lvl_small_kernel<Op>), dim3(small_grid), dim3(kSmallBlock), 0, s, p->ctl,
-                       op);
-    hipLaunchKernelGGL((lvl_combine_kernel<Op>), dim3((kWideReduceMaxNi * 8 + 255) / 256),
-                       dim3(256), 0, s, p->ctl, op, 1);
-    hipLaunchKernelGGL((lvl_combine_kernel<Op>), dim3((p->N + 255) / 256), dim3(256), 0, s,
-                       p->ctl, op, 0);
-#define TUPAN_LVL_SYM(S)                                                                     \
-    if (p->sym_grid[op][S])                                                                  \
-        hipLaunchKernelGGL((lvl_sym_kernel<Op, S>), dim3(p->sym_grid[op][S]),                \
-                           dim3(kSymBlock), 0, s, p->ctl, op);
+    hipLaunchKernelGGL((lvl_small_kernel<Op>), dim3(g[kCandSmall]), dim3(kSmallBlock), 0, s,
+                       p->ctl, op);
+#define TUPAN_LVL_SYM(S)                                                                \
+    if (g[kCandSym + S])                                                                \
+        hipLaunchKernelGGL((lvl_sym_kernel<Op, S>), dim3(g[kCandSym + S]), dim3(kSymBlock), 0, \
+                           s, p->ctl, op);
     TUPAN_LVL_SYM(0)
     TUPAN_LVL_SYM(1)
     TUPAN_LVL_SYM(2)
 #undef TUPAN_LVL_SYM
-    if (p->sym_grid[op][0] || p->sym_grid[op][1] || p->sym_grid[op][2])
-        hipLaunchKernelGGL((lvl_sym_reduce_kernel<Op>), dim3((p->N + kWave - 1) / kWave),
-                           dim3(kSymReduceWaves * kWave), 0, s, p->ctl, op);
+}
+
+template <class OpT, class OpA>
+int lvl_enqueue_pair_workers(const LevelsPlan* p, hipStream_t s)
+{
+    lvl_enqueue_op<OpT>(p, 0, s);
+    lvl_enqueue_op<OpA>(p, 1, s);
+    const int wide = p->N < kWideReduceMaxNi ? p->N : kWideReduceMaxNi;
+    hipLaunchKernelGGL((lvl_combine_kernel<OpT, OpA, true>), dim3((wide * 8 + 255) / 256),
+                       dim3(256), 0, s, p->ctl);
+    if (p->N > kWideReduceMaxNi)
+        hipLaunchKernelGGL((lvl_combine_kernel<OpT, OpA, false>), dim3((p->N + 255) / 256),
+                           dim3(256), 0, s, p->ctl);
+    bool sym = false;
+    for (int op = 0; op < 2; ++op)
+        for (int k = kCandSym; k < kNumCands; ++k) sym = sym || p->gmax[op][k] > 0;
+    if (sym)
+        hipLaunchKernelGGL((lvl_sym_reduce_kernel<OpT, OpA>), dim3((p->N + kWave - 1) / kWave),
+                           dim3(kSymReduceWaves * kWave), 0, s, p->ctl);
     return check_launch("levels pair workers");
 }
 
@@ -1522,13 +1582,12 @@ int sia_levels_enqueue(void* plan, int begin, int nslots, void* stream)
     const int ng = (p->N + 255) / 256;
     for (int k = 0; k < nslots; ++k) {
         hipLaunchKernelGGL(lvl_sched_kernel, dim3(1), dim3(64), 0, s, p->ctl);
-        int rc = p->tstep_mode == TUPAN_MODE_SPLIT32
-                     ? lvl_enqueue_pair_workers<OpSplitTstep>(p, 0, s)
-                     : lvl_enqueue_pair_workers<OpTstep<Fast64>>(p, 0, s);
-        if (rc == TUPAN_OK)
-            rc = p->acc_mode == TUPAN_MODE_SPLIT32
-                     ? lvl_enqueue_pair_workers<OpSplitAcc>(p, 1, s)
-                     : lvl_enqueue_pair_workers<OpAcc<Fast64>>(p, 1, s);
+        const bool st = p->tstep_mode == TUPAN_MODE_SPLIT32;
+        const bool sa = p->acc_mode == TUPAN_MODE_SPLIT32;
+        int rc = st ? (sa ? lvl_enqueue_pair_workers<OpSplitTstep, OpSplitAcc>(p, s)
+                          : lvl_enqueue_pair_workers<OpSplitTstep, OpAcc<Fast64>>(p, s))
+                    : (sa ? lvl_enqueue_pair_workers<OpTstep<Fast64>, OpSplitAcc>(p, s)
+                          : lvl_enqueue_pair_workers<OpTstep<Fast64>, OpAcc<Fast64>>(p, s));
         if (rc != TUPAN_OK) return rc;
         hipLaunchKernelGGL(lvl_part_count_kernel, dim3(nb), dim3(256), 0, s, p->ctl);
         hipLaunchKernelGGL(lvl_part_scan_kernel, dim3(1), dim3(1024), 0, s, p->ctl);

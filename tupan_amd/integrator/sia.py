@@ -582,7 +582,8 @@ class DeviceLevels(object):
 
     STATUS = {1: "Kepler solver failure", 2: "more than 64 levels",
               3: "more than 2^20 level visits",
-              4: "operation queue overflow", 16: "scheduler bound",
+              4: "operation queue overflow", 8: "no worker for a call",
+              16: "scheduler bound",
               32: "no valid step size"}
 
     def __init__(self, sia, slots=256):
