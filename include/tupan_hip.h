@@ -425,7 +425,13 @@ int tupan_kepler_pairs(size_t npairs, const int *idx,
  *   log    NULL or a device log of the near pairs' first solves
  *   counters  NULL or 5 device counters: solves, Laguerre steps,
  *          subdivisions, leapfrog pairs, guess fallbacks
- *   near_pairs  NULL or host int: near pairs listed (-1: one-pass form)
+ *   near_pairs  NULL or host int: near pairs, at most 32 of each list entry
+ *          (a particle and a share of its partners): the log entries of a
+ *          call with one, and the list capacity that tupan_sakura_graph
+ *          needs at most (-1: one-pass form).  A pair of a set with itself
+ *          counts from both sides
+ * Near pairs of an entry beyond the first 32 are solved from the plain guess
+ * and are not logged.
  * net or log imply the two-pass form.  One host synchronisation per call
  * (the near-pair count). */
 typedef struct {

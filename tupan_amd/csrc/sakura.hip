@@ -30,12 +30,12 @@ struct SakuraArgs {
     unsigned long long* counters;
     int* status;
     // two-pass form (null in the one-pass form): per (j-split, i) the count
-    // of deferred near pairs and their j indices (near_slots slots each)
+    // of deferred near pairs and their j indices (kNearSlots slots each)
     int* near_count;
     int* near_j;
     // when set, dt is read from device memory (device-driven steps)
     const double* dt_dev;
-    int near_slots;  // list slots per entry
+    int whole;  // over-full entries are solved whole (kNearSlots)
     // symmetric far pass: blocks of the set and particles per block (0: the
     // tile form, whose entry (s, i) covers the j-range of split s)
     int nb, bi;
@@ -46,16 +46,29 @@ __device__ __forceinline__ double sakura_dt(const SakuraArgs& a)
     return a.dt_dev ? *a.dt_dev : a.dt;
 }
 
-// Near pairs listed per entry; entries with more are solved by
-// near_overflow_kernel.  An entry is an i and the partners one wave met it
-// with: a j-split in the tile form, fewer in the symmetric form.
+// List slots of an entry.  An entry is an i and the partners one wave met it
+// with: a j-split in the tile form, fewer in the symmetric form.  An entry
+// with more near pairs is over-full, and near_overflow_kernel solves the
+// pairs that are not listed, from the plain guess and unlogged: with a guess
+// network or a log all but the first kNearSlots, else all of them (a wave
+// that solves the whole entry has more of its lanes busy, and spares the
+// list: N = 9000, every pair near: 9.6 ms with the first 32 of each entry
+// listed, 5.2 ms whole).  Fewer slots make entries of ordinary states
+// over-full, of whose candidates few are near (N = 6000 with a fifth of the
+// particles slow: 402 us with 32 slots, 735 with 8, 450 in the tile form).
 constexpr int kNearSlots = 32;
-constexpr int kNearSlotsSym = 8;
 
-__device__ __forceinline__ int near_listed(int count, int slots)
+__device__ __forceinline__ int near_listed(int count, int whole)
 {
-    return count > slots ? 0 : count;
+    return count <= kNearSlots ? count : (whole ? 0 : kNearSlots);
 }
+// List items solved at a time (0.9 GiB of items and contributions): a state
+// of many near pairs lists up to kNearSlots per entry, 1.4e9 in all.
+constexpr int kNearWindow = 1 << 24;
+// Largest list capacity with which a graph-safe call takes the symmetric
+// form (3.5 GiB); its caller doubles a capacity that overflowed, and the
+// tile form, with fewer entries, fits beyond.
+constexpr int kSymGraphList = 1 << 26;
 // Calls with at least this many pairs take the two-pass form by default.
 constexpr double kTwoPassPairs = 4194304.0;
 // i-particles per thread in the far-pair pass (independent dependency
@@ -272,7 +285,7 @@ __global__ __launch_bounds__(BLOCK) void sakura_far_kernel(SakuraArgs a)
         Op::load_i(a, {}, valid[w] ? i : a.ni - 1, r[w]);
         Op::zero(acc[w]);
         const size_t entry = static_cast<size_t>(g.jsplit) * a.ni + (valid[w] ? i : 0);
-        slots[w] = a.near_j + entry * a.near_slots;
+        slots[w] = a.near_j + entry * kNearSlots;
         ndef[w] = 0;
     }
     const int j0 = g.jsplit * a.jchunk;
@@ -294,9 +307,9 @@ __global__ __launch_bounds__(BLOCK) void sakura_far_kernel(SakuraArgs a)
                 double p[3] = {p0[0], p0[1], p0[2]};
                 double v[3] = {v0[0], v0[1], v0[2]};
                 if (!kep::drift_twobody_far_t<FLAG>(r[w].dt, m, e2, p, v, acc[w].c)) {
-                    // near pair; an entry with more than its slots goes to
-                    // near_overflow_kernel whole
-                    if (ndef[w] < a.near_slots) slots[w][ndef[w]] = jt + k;
+                    // near pair: the first kNearSlots go to the list, the
+                    // rest to near_overflow_kernel
+                    if (ndef[w] < kNearSlots) slots[w][ndef[w]] = jt + k;
                     ++ndef[w];
                     continue;
                 }
@@ -425,13 +438,13 @@ __global__ __launch_bounds__(kWave* kSymFarWaves, 2) void sakura_far_sym_kernel(
                 double p[3] = {p0[0], p0[1], p0[2]};
                 double v[3] = {v0[0], v0[1], v0[2]};
                 if (!kep::drift_twobody_far_t<FLAG>(dt, m, e2, p, v, c)) {
-                    if (ndef[w] < a.near_slots)
-                        a.near_j[(static_cast<size_t>(chunk) * n + i) * a.near_slots + ndef[w]] =
+                    if (ndef[w] < kNearSlots)
+                        a.near_j[(static_cast<size_t>(chunk) * n + i) * kNearSlots + ndef[w]] =
                             j0 + jl;
                     ++ndef[w];
                     if (d > 0) {
-                        if (jdef < a.near_slots)
-                            a.near_j[(jentry + jl) * a.near_slots + jdef] = i;
+                        if (jdef < kNearSlots)
+                            a.near_j[(jentry + jl) * kNearSlots + jdef] = i;
                         ++jdef;
                     }
                     continue;
@@ -522,7 +535,7 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* lds, int& block_
     return incl - v;
 }
 
-__global__ __launch_bounds__(kScanThreads) void near_block_sums_kernel(int n, int slots,
+__global__ __launch_bounds__(kScanThreads) void near_block_sums_kernel(int n, int whole,
                                                                        const int* count,
                                                                        int* bsum, int* bover)
 {
@@ -533,8 +546,8 @@ __global__ __launch_bounds__(kScanThreads) void near_block_sums_kernel(int n, in
         const int e = base + q;
         if (e < n) {
             const int c = count[e];
-            sum += near_listed(c, slots);
-            ov += c > slots;
+            sum += near_listed(c, whole);
+            ov += c > kNearSlots;
         }
     }
     int tot_s, tot_o;
@@ -577,7 +590,7 @@ __global__ __launch_bounds__(kScanThreads) void near_block_offsets_kernel(int nb
     }
 }
 
-__global__ __launch_bounds__(kScanThreads) void near_offsets_kernel(int n, int slots,
+__global__ __launch_bounds__(kScanThreads) void near_offsets_kernel(int n, int whole,
                                                                     const int* count,
                                                                     const int* boff, int* off,
                                                                     int* total, int* over_list)
@@ -589,7 +602,7 @@ __global__ __launch_bounds__(kScanThreads) void near_offsets_kernel(int n, int s
     for (int q = 0; q < 4; ++q) {
         const int e = base + q;
         c[q] = e < n ? count[e] : 0;
-        sum += near_listed(c[q], slots);
+        sum += near_listed(c[q], whole);
     }
     int tot;
     int run = boff[blockIdx.x] + block_exclusive_scan(sum, lds, tot);
@@ -597,26 +610,36 @@ __global__ __launch_bounds__(kScanThreads) void near_offsets_kernel(int n, int s
         const int e = base + q;
         if (e >= n) break;
         off[e] = run;
-        run += near_listed(c[q], slots);
-        if (c[q] > slots) over_list[atomicAdd(total + 2, 1)] = e;
+        run += near_listed(c[q], whole);
     }
+    // the over-full entries, one atomic per block
+    int ov = 0;
+    for (int q = 0; q < 4; ++q) ov += c[q] > kNearSlots;  // 0 past the last entry
+    __shared__ int over_base;
+    int mine = block_exclusive_scan(ov, lds, tot);
+    if (tot == 0) return;
+    if (threadIdx.x == 0) over_base = atomicAdd(total + 2, tot);
+    __syncthreads();
+    for (int q = 0; q < 4; ++q)
+        if (c[q] > kNearSlots) over_list[over_base + mine++] = base + q;
 }
 
 // Near-pair list: item = (i, partner), grouped by entry, in the order met.
-// Items at or beyond `cap` are not written (a call whose list is longer
-// than its capacity is flagged by near_capacity_kernel).
-__global__ __launch_bounds__(256) void near_compact_kernel(int n, int ni, int slots,
-                                                           const int* count, const int* off,
-                                                           const int* near_j,
-                                                           int2* items, int cap)
+// `items` holds the window of `cap` items from `base` on; items outside it
+// are not written (in a graph-safe call, whose one window is its capacity,
+// near_capacity_kernel flags a longer list).
+__global__ __launch_bounds__(256) void near_compact_kernel(int n, int ni, int whole,
+                                                           const int* count,
+                                                           const int* off, const int* near_j,
+                                                           int2* items, int base, int cap)
 {
     const int e = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= n) return;
-    const int c = near_listed(count[e], slots);
-    const int o = off[e];
+    const int c = near_listed(count[e], whole);
+    const int o = off[e] - base;
     const int i = e % ni;
-    for (int k = 0; k < c && o + k < cap; ++k)
-        items[o + k] = make_int2(i, near_j[static_cast<size_t>(e) * slots + k]);
+    for (int k = max(0, -o); k < c && o + k < cap; ++k)
+        items[o + k] = make_int2(i, near_j[static_cast<size_t>(e) * kNearSlots + k]);
 }
 
 // Capacity check of the graph-safe form: status bit 2 when the near-pair
@@ -626,11 +649,11 @@ __global__ void near_capacity_kernel(const int* total, int cap, int* status)
     if (threadIdx.x == 0 && total[0] > cap && status) atomicOr(status, 2);
 }
 
-// One near pair, item t of the list: the pair's drift (from the learned
-// guess when `guess` is set and usable), its six contributions (contrib is
-// SoA [6][nitems]) and, with a log, the first stage's features, the learned
-// target and the pair's Laguerre steps.
-__device__ __forceinline__ void near_pair(const SakuraArgs& a, int t, int nitems,
+// One near pair, item t of the window that starts at item `base` of the
+// list: the pair's drift (from the learned guess when `guess` is set and
+// usable), its six contributions (contrib [nitems][6]) and, with a log, the
+// first stage's features, the learned target and the pair's Laguerre steps.
+__device__ __forceinline__ void near_pair(const SakuraArgs& a, int t, int base,
                                           const int2* items, double* contrib, bool guess,
                                           float d, const SolveLogDev& log, kep::Counters& c)
 {
@@ -650,18 +673,15 @@ __device__ __forceinline__ void near_pair(const SakuraArgs& a, int t, int nitems
         gs.use = d == d && d > -0.9f && d < 8.0f;
         gs.delta = static_cast<double>(d);
     }
-    const bool logging = log.target != nullptr && t < log.capacity;
+    const bool logging = log.target != nullptr && base + t < log.capacity;
     double s_conv = __builtin_nan("");
     kep::drift_twobody(sakura_dt(a), a.flag, m, e2, p, v, c, guess ? &gs : nullptr,
                        logging ? &s_conv : nullptr);
     const double mu = mj / m;
-    const size_t n = static_cast<size_t>(nitems);
-    contrib[0 * n + t] = mu * (p[0] - p0[0]);
-    contrib[1 * n + t] = mu * (p[1] - p0[1]);
-    contrib[2 * n + t] = mu * (p[2] - p0[2]);
-    contrib[3 * n + t] = mu * (v[0] - v0[0]);
-    contrib[4 * n + t] = mu * (v[1] - v0[1]);
-    contrib[5 * n + t] = mu * (v[2] - v0[2]);
+    double2* out = reinterpret_cast<double2*>(contrib) + 3 * static_cast<size_t>(t);
+    out[0] = make_double2(mu * (p[0] - p0[0]), mu * (p[1] - p0[1]));
+    out[1] = make_double2(mu * (p[2] - p0[2]), mu * (v[0] - v0[0]));
+    out[2] = make_double2(mu * (v[1] - v0[1]), mu * (v[2] - v0[2]));
     if (logging) {
         double q[3] = {p0[0], p0[1], p0[2]};
         const double dts = kep::first_stage(sakura_dt(a), a.flag, q, v0);
@@ -671,12 +691,13 @@ __device__ __forceinline__ void near_pair(const SakuraArgs& a, int t, int nitems
         if (kep::solve_setup(dts, m, e2, q, v0, k, s0, &f) && s_conv == s_conv)
             target = static_cast<float>(s_conv * k[1] / k[0] - 1);
         const size_t cap = static_cast<size_t>(log.capacity);
-        log.features[0 * cap + t] = f.tau;
-        log.features[1 * cap + t] = f.sigma;
-        log.features[2 * cap + t] = f.kappa;
-        log.features[3 * cap + t] = f.eps;
-        log.target[t] = target;
-        log.iterations[t] = static_cast<int>(c.iters);
+        const size_t g = static_cast<size_t>(base) + t;
+        log.features[0 * cap + g] = f.tau;
+        log.features[1 * cap + g] = f.sigma;
+        log.features[2 * cap + g] = f.kappa;
+        log.features[3 * cap + g] = f.eps;
+        log.target[g] = target;
+        log.iterations[g] = static_cast<int>(c.iters);
     }
 }
 
@@ -698,7 +719,7 @@ __device__ __forceinline__ void near_flush(const SakuraArgs& a, bool valid,
 // Pass 2: one near pair per thread.  With `delta` the first solve of the
 // pair starts from the learned guess (kepler.h: Guess).
 __global__ __launch_bounds__(128) void sakura_near_kernel(SakuraArgs a, int nitems,
-                                                          const int* nitems_dev,
+                                                          const int* nitems_dev, int base,
                                                           const int2* items, double* contrib,
                                                           const float* delta, SolveLogDev log,
                                                           unsigned long long* bank)
@@ -710,8 +731,8 @@ __global__ __launch_bounds__(128) void sakura_near_kernel(SakuraArgs a, int nite
     const bool valid = t < count;
     kep::Counters c;
     if (valid)
-        near_pair(a, t, nitems, items, contrib, delta != nullptr, delta ? delta[t] : 0.f, log,
-                  c);
+        near_pair(a, t, base, items, contrib, delta != nullptr, delta ? delta[t] : 0.f,
+                  log, c);
     near_flush(a, valid, c, bank);
 }
 
@@ -721,7 +742,7 @@ __global__ __launch_bounds__(128) void sakura_near_kernel(SakuraArgs a, int nite
 // with the stand-alone inference kernel's arithmetic (mlp_wave.h), then
 // solves its pairs from the guesses.  The packed network is staged in LDS.
 __global__ __launch_bounds__(128, 2) void sakura_near_learned_kernel(SakuraArgs a, int nitems,
-                                                                  const int2* items,
+                                                                  int base, const int2* items,
                                                                   double* contrib,
                                                                   const NetPacked* net,
                                                                   SolveLogDev log,
@@ -763,75 +784,107 @@ __global__ __launch_bounds__(128, 2) void sakura_near_learned_kernel(SakuraArgs 
     // live across the network (register pressure)
     __asm__ volatile("" ::: "memory");
     kep::Counters c;
-    if (valid) near_pair(a, t, nitems, items, contrib, true, d, log, c);
+    if (valid) near_pair(a, t, base, items, contrib, true, d, log, c);
     near_flush(a, valid, c, bank);
 }
 
-// Pass 3: add each (split, i)'s near contributions, in list order, to its
-// far partial sum.
-__global__ __launch_bounds__(256) void near_add_kernel(int n, int ni, int nitems, int slots,
-                                                       const int* count, const int* off,
+// Pass 3: add each entry's near contributions, in list order, to its far
+// partial sum (those in the window of nitems items from `base` on; the
+// windows come in order).
+__global__ __launch_bounds__(256) void near_add_kernel(int n, int ni, int nitems, int base,
+                                                       int whole, const int* count, const int* off,
                                                        const double* contrib, double* partial)
 {
     const int e = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= n) return;
-    const int c = near_listed(count[e], slots);
-    if (c == 0) return;
-    const int o = off[e];
+    const int c = near_listed(count[e], whole);
+    const int o = off[e] - base;
+    const int q0 = max(0, -o), q1 = min(c, nitems - o);
+    if (q0 >= q1) return;
     const int split = e / ni;
     const int i = e % ni;
     double* part = partial + static_cast<size_t>(split) * 6 * ni;
-    for (int k = 0; k < 6; ++k) {
-        double sum = part[static_cast<size_t>(k) * ni + i];
-        for (int q = 0; q < c && o + q < nitems; ++q)
-            sum += contrib[static_cast<size_t>(k) * nitems + o + q];
-        part[static_cast<size_t>(k) * ni + i] = sum;
+    // eight items' loads in flight: an entry of many items is a chain of
+    // memory latency otherwise
+    constexpr int kBatch = 8;
+    double sum[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) sum[k] = part[static_cast<size_t>(k) * ni + i];
+    const double2* src = reinterpret_cast<const double2*>(contrib) + 3 * static_cast<long long>(o);
+    for (int q = q0; q < q1; q += kBatch) {
+        double2 v[kBatch][3];
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                v[b][k] = q + b < q1 ? src[3 * (q + b) + k] : make_double2(0.0, 0.0);
+        }
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b) {
+            if (q + b >= q1) break;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                sum[2 * k] += v[b][k].x;
+                sum[2 * k + 1] += v[b][k].y;
+            }
+        }
     }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) part[static_cast<size_t>(k) * ni + i] = sum[k];
 }
 
-// The partners of an entry: how many candidates, and candidate k (a particle
-// index, or -1 where the last block ends).
+// The partners of an entry in the order the far pass met them: how many
+// candidates, and candidate k (a particle index, or -1 past the set's end).
 struct Partners {
-    int first, count;   // tile form and j entries: consecutive particles
-    int row, t0;        // i entries of the symmetric form: tiles from t0 on
+    int first, count;
+    int kind;       // 0 tile form, 1 i entry, 2 j entry of the symmetric form
+    int t0, lane;   // i entry: first tile; the lane that held the particle
 };
 
 __device__ __forceinline__ Partners entry_partners(const SakuraArgs& a, int split, int i)
 {
     if (a.nb == 0) {
         const int j0 = split * a.jchunk;
-        return {j0, min(a.nj, j0 + a.jchunk) - j0, -1, 0};
+        return {j0, min(a.nj, j0 + a.jchunk) - j0, 0, 0, 0};
     }
     const int block = i / a.bi;
+    const int lane = i % kWave;  // blocks are whole waves
     const int nchunk = a.nsplit - a.nb / 2;
     if (split >= nchunk) {
         int row = block - (split - nchunk + 1);
         if (row < 0) row += a.nb;
-        return {row * a.bi, a.bi, -1, 0};
+        return {row * a.bi, a.bi, 2, 0, lane};
     }
     const int tiles = sym_row_tiles(a.nb, block, a.bi / kWave);
     const int t0 = static_cast<int>(static_cast<long long>(tiles) * split / nchunk);
     const int t1 = static_cast<int>(static_cast<long long>(tiles) * (split + 1) / nchunk);
-    return {0, (t1 - t0) * kWave, block, t0};
+    return {block, (t1 - t0) * kWave, 1, t0, lane};
 }
 
 __device__ __forceinline__ int partner(const SakuraArgs& a, const Partners& P, int k)
 {
     if (k >= P.count) return -1;
     int j = P.first + k;
-    if (P.row >= 0) {
-        const int t = P.t0 + k / kWave, tpb = a.bi / kWave;
-        int block = P.row + t / tpb;
+    const int sh = a.bi == 4 * kWave ? 2 : 1;  // W = 4 or 2 particles per lane
+    if (P.kind == 1) {
+        // tile after tile, in step s the particle s lanes below
+        const int t = P.t0 + k / kWave;
+        int block = P.first + (t >> sh);
         if (block >= a.nb) block -= a.nb;
-        j = block * a.bi + (t % tpb) * kWave + k % kWave;
+        j = block * a.bi + (t & ((1 << sh) - 1)) * kWave + ((P.lane - k) & (kWave - 1));
+    } else if (P.kind == 2) {
+        // in step s the W particles of the lane s above
+        j = P.first + (k & ((1 << sh) - 1)) * kWave + ((P.lane + (k >> sh)) & (kWave - 1));
     }
     return j < a.nj ? j : -1;
 }
 
 // Entries with more near pairs than list slots, one wave per entry: the
-// wave walks the entry's partners in chunks of 64 (one per lane), solves the
-// near ones in parallel and adds the chunk's contributions to the partial
-// sum through a fixed shuffle tree (deterministic).
+// wave walks the entry's partners in chunks of 64 (one per lane), ranks the
+// near ones of the chunk in the order met with a ballot, solves those that
+// are not listed (in parallel, one per lane), and adds the
+// chunk's contributions to the partial sum through a fixed shuffle tree
+// (deterministic).
 __device__ __forceinline__ void overflow_entry(const SakuraArgs& a, int e, int lane,
                                                kep::Counters& c)
 {
@@ -839,6 +892,7 @@ __device__ __forceinline__ void overflow_entry(const SakuraArgs& a, int e, int l
     const int i = e % a.ni;
     const Partners P = entry_partners(a, split, i);
     double d[6] = {0, 0, 0, 0, 0, 0};
+    int seen = 0;  // near pairs before this chunk
     for (int kb = 0; kb < P.count; kb += kWave) {
         const int j = partner(a, P, kb + lane);
         const int jj = j < 0 ? i : j;
@@ -854,8 +908,11 @@ __device__ __forceinline__ void overflow_entry(const SakuraArgs& a, int e, int l
         kep::Counters scratch;
         const bool near =
             j >= 0 && !kep::drift_twobody_far(sakura_dt(a), a.flag, m, e2, p, v, scratch);
+        const unsigned long long mask = __ballot(near);
+        const int rank = seen + __popcll(mask & ((1ull << lane) - 1ull));
+        seen += __popcll(mask);
         double cd[6] = {0, 0, 0, 0, 0, 0};
-        if (near) {
+        if (near && (a.whole || rank >= kNearSlots)) {
             p[0] = p0[0]; p[1] = p0[1]; p[2] = p0[2];
             v[0] = v0[0]; v[1] = v0[1]; v[2] = v0[2];
             kep::drift_twobody(sakura_dt(a), a.flag, m, e2, p, v, c);
@@ -899,13 +956,14 @@ __global__ __launch_bounds__(64) void near_overflow_kernel(SakuraArgs a, const i
 // The symmetric far pass's plan for a set against itself; false where the
 // tile form takes the call: up to kSymFarAbove particles, where it spreads
 // the work finer (n = 4096: 244 us, 253 symmetric; 6000: 321 and 264 us), and
-// where the entries' sums, counts and lists pass kSymMaxBytes (n = 150000).
+// where the entries' sums, counts and lists pass kSymFarMaxBytes (n = 150000).
 // Four particles per lane above kSymFarW4Above (n = 12000: 543 us with four,
 // 498 with two; 24001: 1507 and 1556 us; 65536: 9.50 and 9.74 ms).  Chunks
 // per row: at least two waves per SIMD, and of the counts up to four times
 // that the one whose busiest SIMD has the least to do, a wave's fixed cost
 // counted as a quarter of a tile.
 constexpr int kSymFarAbove = 5120, kSymFarW4Above = 20480;
+constexpr size_t kSymFarMaxBytes = static_cast<size_t>(8) << 30;
 
 static bool sakura_sym_plan(SakuraArgs& a, int cu, unsigned* grid)
 {
@@ -931,13 +989,12 @@ static bool sakura_sym_plan(SakuraArgs& a, int cu, unsigned* grid)
     }
     const size_t slots = static_cast<size_t>(nchunk) + nb / 2;
     const size_t nent = slots * a.ni;
-    constexpr size_t kEntryBytes = 6 * sizeof(double) + (3 + kNearSlotsSym) * sizeof(int);
-    if (nent * kEntryBytes > kSymMaxBytes) return false;
+    constexpr size_t kEntryBytes = 6 * sizeof(double) + (3 + kNearSlots) * sizeof(int);
+    if (nent * kEntryBytes > kSymFarMaxBytes) return false;
     a.nb = nb;
     a.bi = bi;
     a.nsplit = static_cast<int>(slots);
     a.jchunk = 0;
-    a.near_slots = kNearSlotsSym;
     *grid = (static_cast<unsigned>(nb) * static_cast<unsigned>(nchunk) + kSymFarWaves - 1) /
             kSymFarWaves;
     return true;
@@ -1001,10 +1058,11 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
     }
     a.nsplit = L.nsplit;
     a.jchunk = L.jchunk;
-    a.near_slots = kNearSlots;
+    a.whole = !opt.net && !opt.log.target;
     opt.near_pairs = -1;
     unsigned grid = static_cast<unsigned>(L.nblock_i) * static_cast<unsigned>(L.nsplit);
-    if (two_pass && sakura_sym_plan(a, dev.cu_count, &grid)) nent = static_cast<size_t>(a.nsplit) * ni;
+    if (two_pass && opt.graph_capacity <= kSymGraphList && sakura_sym_plan(a, dev.cu_count, &grid))
+        nent = static_cast<size_t>(a.nsplit) * ni;
     const unsigned rg = static_cast<unsigned>((a.ni + 255) / 256);
     if (!two_pass) {
         if (L.nsplit > 1) {
@@ -1031,7 +1089,7 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
     const size_t b_blk = up(static_cast<size_t>(nb) * sizeof(int));
     const size_t b_tot = 256;
     const size_t b_bank = up(kBankSlots * kBankStride * sizeof(unsigned long long));
-    const size_t b_slots = up(nent * a.near_slots * sizeof(int));
+    const size_t b_slots = up(nent * kNearSlots * sizeof(int));
     char* w1 = static_cast<char*>(
         workspace(b_part + 3 * b_cnt + 2 * b_blk + b_tot + b_bank + b_slots, s, 1));
     if (!w1) return set_error(TUPAN_ERR_ALLOC, "workspace allocation failed");
@@ -1069,11 +1127,11 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
     timing_end(s);
     timing_begin(s);
     hipLaunchKernelGGL(near_block_sums_kernel, dim3(nb), dim3(kScanThreads), 0, s, n,
-                       a.near_slots, a.near_count, bsum, bover);
+                       a.whole, a.near_count, bsum, bover);
     hipLaunchKernelGGL(near_block_offsets_kernel, dim3(1), dim3(kScanThreads), 0, s, nb, bsum,
                        bover, total_dev, bank);
     hipLaunchKernelGGL(near_offsets_kernel, dim3(nb), dim3(kScanThreads), 0, s, n,
-                       a.near_slots, a.near_count, bsum, near_off, total_dev, over_list);
+                       a.whole, a.near_count, bsum, near_off, total_dev, over_list);
     const unsigned eg = static_cast<unsigned>((n + 255) / 256);
     if (graph) {
         // No host synchronisation: the list gets the caller's capacity, the
@@ -1089,14 +1147,14 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
         double* contrib = reinterpret_cast<double*>(w2 + b_items);
         hipLaunchKernelGGL(near_capacity_kernel, dim3(1), dim3(64), 0, s, total_dev, cap, status);
         hipLaunchKernelGGL(near_compact_kernel, dim3(eg), dim3(256), 0, s, n, a.ni,
-                           a.near_slots, a.near_count, near_off, a.near_j, items, cap);
+                           a.whole, a.near_count, near_off, a.near_j, items, 0, cap);
         hipLaunchKernelGGL(sakura_near_kernel, dim3((cap + 127) / 128), dim3(128), 0, s, a, cap,
-                           total_dev, items, contrib, nullptr, opt.log, bank);
+                           total_dev, 0, items, contrib, nullptr, opt.log, bank);
         if (bank)
             hipLaunchKernelGGL(near_bank_flush_kernel, dim3(1), dim3(64), 0, s, bank, a.counters,
                                opt.fallbacks);
-        hipLaunchKernelGGL(near_add_kernel, dim3(eg), dim3(256), 0, s, n, a.ni, cap,
-                           a.near_slots, a.near_count, near_off, contrib, a.partial);
+        hipLaunchKernelGGL(near_add_kernel, dim3(eg), dim3(256), 0, s, n, a.ni, cap, 0,
+                           a.whole, a.near_count, near_off, contrib, a.partial);
         hipLaunchKernelGGL(near_overflow_kernel, dim3(kOverflowWaves), dim3(kWave), 0, s, a,
                            over_list, 0, total_dev + 1);
         hipLaunchKernelGGL((reduce_kernel<OpSakura>), dim3(rg), dim3(256), 0, s, a);
@@ -1111,32 +1169,37 @@ int sakura_call_ex(size_t ni, const double* const* ip, size_t nj, const double* 
     if (rc == TUPAN_OK) rc = check_hip(hipStreamSynchronize(s), "near-pair count");
     if (rc != TUPAN_OK) return rc;
     const int total = counts[0];
-    opt.near_pairs = total;
+    // min(count, kNearSlots) of every entry
+    opt.near_pairs = total + (a.whole ? kNearSlots * counts[1] : 0);
     if (total > 0) {
-        // workspace slot 2: items and contributions
-        const size_t nt = static_cast<size_t>(total);
+        // workspace slot 2: items and contributions of one window
+        const int window = total < kNearWindow ? total : kNearWindow;
+        const size_t nt = static_cast<size_t>(window);
         const size_t b_items = up(nt * sizeof(int2));
         const size_t b_con = up(nt * 6 * sizeof(double));
         char* w2 = static_cast<char*>(workspace(b_items + b_con, s, 2));
         if (!w2) return set_error(TUPAN_ERR_ALLOC, "workspace allocation failed");
         int2* items = reinterpret_cast<int2*>(w2);
         double* contrib = reinterpret_cast<double*>(w2 + b_items);
-        hipLaunchKernelGGL(near_compact_kernel, dim3(eg), dim3(256), 0, s, n, a.ni,
-                           a.near_slots, a.near_count, near_off, a.near_j, items, total);
-        const unsigned ig = static_cast<unsigned>((total + 127) / 128);
-        if (opt.net) {
-            hipLaunchKernelGGL(sakura_near_learned_kernel, dim3(ig), dim3(128), 0, s, a, total,
-                               items, contrib, static_cast<const NetPacked*>(opt.net), opt.log,
-                               bank);
-        } else {
-            hipLaunchKernelGGL(sakura_near_kernel, dim3(ig), dim3(128), 0, s, a, total, nullptr,
-                               items, contrib, nullptr, opt.log, bank);
+        for (int base = 0; base < total; base += window) {
+            const int cnt = total - base < window ? total - base : window;
+            hipLaunchKernelGGL(near_compact_kernel, dim3(eg), dim3(256), 0, s, n, a.ni,
+                               a.whole, a.near_count, near_off, a.near_j, items, base, cnt);
+            const unsigned ig = static_cast<unsigned>((cnt + 127) / 128);
+            if (opt.net) {
+                hipLaunchKernelGGL(sakura_near_learned_kernel, dim3(ig), dim3(128), 0, s, a, cnt,
+                                   base, items, contrib, static_cast<const NetPacked*>(opt.net),
+                                   opt.log, bank);
+            } else {
+                hipLaunchKernelGGL(sakura_near_kernel, dim3(ig), dim3(128), 0, s, a, cnt, nullptr,
+                                   base, items, contrib, nullptr, opt.log, bank);
+            }
+            hipLaunchKernelGGL(near_add_kernel, dim3(eg), dim3(256), 0, s, n, a.ni, cnt, base,
+                               a.whole, a.near_count, near_off, contrib, a.partial);
         }
         if (bank)
             hipLaunchKernelGGL(near_bank_flush_kernel, dim3(1), dim3(64), 0, s, bank, a.counters,
                                opt.fallbacks);
-        hipLaunchKernelGGL(near_add_kernel, dim3(eg), dim3(256), 0, s, n, a.ni, total,
-                           a.near_slots, a.near_count, near_off, contrib, a.partial);
     }
     if (counts[1] > 0) {
         hipLaunchKernelGGL(near_overflow_kernel, dim3(counts[1]), dim3(kWave), 0, s, a,

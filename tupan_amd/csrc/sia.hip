@@ -745,8 +745,7 @@ int sia_update_call(int kind, size_t n, void* const* arrays, double h, void* str
 // scheduler wrote and exits unless the slot is its own, so the launch
 // sequence is fixed and a run of slots can be captured as one HIP graph and
 // replayed until the step's stack is empty.  A slot costs its launches, most
-// of them empty (about 2 us each, more with thousands of workgroups): a
-// worker no call can reach is not launched, and grids are no larger than the
+// of them empty: a worker no call can reach is not launched, and grids are no larger than the
 // largest plan (sia21h step, FP64, N = 3000: 464 ms with every shape of the
 // table at its target's grid, 288 ms; N = 12000: 1055 and 760 ms).
 //

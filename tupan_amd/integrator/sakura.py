@@ -105,7 +105,7 @@ class DeviceSakura(object):
             self.native.check(rc, "tupan_sakura_ex")
             most = max(most, npairs.value)
         self.status.zero_()
-        self.capacity = max(4 * most, 4096)
+        self.capacity = max(min(4 * most, 1 << 30), 4096)  # a C int
 
     def launch(self):
         from ..lib.hip_backend import current_stream_handle
