@@ -91,8 +91,10 @@ int tupan_timing_read_each(double *ms, int max, int *count);
  * table entry for (kernel TUPAN_K_*, slot, bucket) picks the shape and the
  * workgroups-per-CU target of the launch planner.  slot: 0 FP64, 1
  * split-FP32, 2 reference-order FP64, 3 float build.  bucket by pair count
- * ni*nj: 0 below 2^25, 1 below 2^30, 2 above; a call whose ni the picked
- * shape would pad by more than a quarter takes bucket 0's entry.  Default:
+ * ni*nj: 0 below 2^25 (2^22 for PNAcc, and for SnapCrackle of 16384 or more
+ * i), 1 below 2^30, 2 above; a call whose ni the picked shape would pad by
+ * more than a quarter takes bucket 0's entry, and a call of 24576 or more i
+ * in bucket 0 aims for twice its workgroups per CU (up to 16).  Default:
  * shape 0, 4 workgroups per CU.  The table is process-wide.  Calls of at
  * most 2^21 pairs with 256 < nj <= 2048 (any mode but reference-order FP64)
  * run a one-launch small-set kernel that does not consult the table, and a

@@ -509,13 +509,31 @@ constexpr int kLightShapeDims[kNumShapes][4] = {
 // to 4 (split AccJerk 300 x 50000, pair kernel: 24 us, 108 at 512 x 2); above,
 // their one i per lane and short j ranges cost up to 1.25 (split AccJerk
 // 9000 x 7000: 89 us, 75 at two per lane; FP64 Acc 15000 x 15500: 196, 166).
-// From 2^30 the widest tiles are level or better.
-__host__ __device__ inline int size_bucket(int ni, int nj)
+// PNAcc, a few hundred operations per pair, fills it from 2^22 on (split
+// 14200 x 659: 93 us with bucket 0's shape, 76 with bucket 1's; 5000 x 5000:
+// 214 and 190), SnapCrackle where there are 16384 i (float 27066 x 575: 49
+// and 38 us; below, 2938 x 6607: 46 and 53).  From 2^30 the widest tiles are
+// level or better.
+enum class Weight { light, snap_crackle, pnacc };
+__host__ __device__ inline int size_bucket(int ni, int nj, Weight w = Weight::light)
 {
     const double pairs = static_cast<double>(ni) * static_cast<double>(nj);
-    if (pairs < 33554432.0) return 0;    // < 2^25
-    if (pairs < 1073741824.0) return 1;  // < 2^30
+    const bool low = w == Weight::pnacc || (w == Weight::snap_crackle && ni >= 16384);
+    if (pairs < (low ? 4194304.0 : 33554432.0)) return 0;  // < 2^22, < 2^25
+    if (pairs < 1073741824.0) return 1;                    // < 2^30
     return 2;
+}
+
+// Workgroups per CU of a call in bucket b.  From 24576 i on (384 one-wave
+// rows) the few splits of bucket 0's target leave some SIMDs a wave more
+// than others, a third of the time of so short a call: twice the target
+// there (FP64 Tstep 27066 x 575: 44 -> 33 us, FP64 AccJerk 35000 x 400: 40
+// -> 34 us); below it costs up to a sixth (float NREG X 11680 x 736: 18 us,
+// 22 at twice).
+constexpr int kManyRows = 24576;
+__host__ __device__ inline int bucket_wg(int b, int ni, int wg)
+{
+    return b == 0 && ni >= kManyRows && wg < 16 ? 2 * wg : wg;
 }
 
 // A shape whose workgroups would pad ni by more than a quarter (few i against

@@ -396,11 +396,14 @@ static int launch_tuned(const Launcher<Op> (&table)[kShapes], int kernel, int sl
 {
     int rc = TUPAN_OK;
     if (run_sym<Op>(a, s, fixed, &rc)) return rc;
-    int b = size_bucket(a.ni, a.nj);
+    int b = size_bucket(a.ni, a.nj,
+                        kernel == K_SNAP_CRACKLE ? Weight::snap_crackle
+                        : kernel == K_PNACC      ? Weight::pnacc
+                                                 : Weight::light);
     const int* d = shape_dims(kernel, g_tune[kernel][slot][b].shape);
     if (pads_rows(a.ni, d[0], d[1])) b = 0;
     const TuneEntry& t = g_tune[kernel][slot][b];
-    return table[t.shape](a, s, t.wg_per_cu, fixed);
+    return table[t.shape](a, s, bucket_wg(b, a.ni, t.wg_per_cu), fixed);
 }
 
 #define TUPAN_RUN(Op, SHAPES, kernel, slot)                                      \

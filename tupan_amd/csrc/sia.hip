@@ -889,7 +889,7 @@ __device__ void lvl_plan_pair(LvlCtl* c, int op, int ilo, int ni, int jlo, int n
     if (pads_rows(ni, kLightShapeDims[c->tshape[op][b]][0], kLightShapeDims[c->tshape[op][b]][1]))
         b = 0;
     const int shape = c->tshape[op][b];
-    const int wg = c->twg[op][b];
+    const int wg = bucket_wg(b, ni, c->twg[op][b]);
     const int BLOCK = kLightShapeDims[shape][0], WPT = kLightShapeDims[shape][1],
               TILE = kLightShapeDims[shape][2];
     const int target = (wg > 0 ? wg : 4) * c->cu_count;
@@ -1391,7 +1391,7 @@ size_t lvl_workers(LvlCtl& h, int n)
         for (int b = 0; b <= last_bucket; ++b) {
             const int s = h.tshape[op][b];
             const int ipb = kLightShapeDims[s][0] * kLightShapeDims[s][1];
-            const int wg = h.twg[op][b] > 0 ? h.twg[op][b] : 4;
+            const int wg = bucket_wg(b, n, h.twg[op][b] > 0 ? h.twg[op][b] : 4);
             const long long target = static_cast<long long>(wg) * h.cu_count;
             const long long nblk = (n + ipb - 1) / ipb;
             // plan_launch: nblock_i * nsplit is at most target + nblock_i, or

@@ -31,14 +31,20 @@ KERNELS = {  # name -> (kernel id, modes)
     "nreg_v": (_native.K_NREG_V, ("fp64", "float32")),
     "pnacc": (_native.K_PNACC, ("fp64", "split32", "float32")),
 }
-# (ni, nj) of the calls timed per size bucket (below 2^25 pairs, below 2^30,
-# above)
-BUCKET_SETS = (
-    ((200, 3000), (64, 16000), (4000, 700), (2000, 2100), (300, 50000),
-     (16000, 700), (4000, 4096)),
-    ((2501, 60000), (9000, 7000), (15000, 15500), (60000, 2500), (30000, 31000)),
-    ((20000, 60000), (65000, 66000)),
-)
+# (ni, nj) of the calls timed, each in its kernel's size bucket
+SETS = ((200, 3000), (64, 16000), (4000, 700), (2000, 2100), (300, 50000),
+        (16000, 700), (4000, 4096), (3000, 50000), (6000, 6000), (9000, 7000),
+        (15000, 15500), (60000, 2500), (30000, 31000), (20000, 60000),
+        (65000, 66000))
+
+
+def size_bucket(name, ni, nj):
+    """The library's bucket of a call (engine.h: size_bucket)."""
+    pairs = ni * nj
+    low = name == "pnacc" or (name == "snap_crackle" and ni >= 16384)
+    if pairs < (1 << 22 if low else 1 << 25):
+        return 0
+    return 1 if pairs < 1 << 30 else 2
 
 
 def cluster(n, seed=0, dtype=torch.float64):
@@ -108,10 +114,11 @@ def tune_pairwise(quick, names, pinned=()):
                "snap_crackle": extensions.SnapCrackle,
                "tstep": extensions.Tstep, "nreg_x": extensions.NREG_X,
                "nreg_v": extensions.NREG_V, "pnacc": extensions.PNAcc}
-    for b, sets in enumerate(BUCKET_SETS[:2] if quick else BUCKET_SETS):
+    for b in range(2 if quick else 3):
         for name, (kid, modes) in KERNELS.items():
             if name not in names:
                 continue
+            sets = [s for s in SETS if size_bucket(name, *s) == b]
             for mode in modes:
                 if (name, mode) in pinned:
                     continue
