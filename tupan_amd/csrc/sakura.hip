@@ -356,15 +356,6 @@ __global__ __launch_bounds__(BLOCK) void sakura_far_kernel(SakuraArgs a)
 // flag -1: N = 16384 1.26 -> 0.84 ms, 65536 19.4 -> 9.5 ms.
 constexpr int kSymFarWaves = 4;
 
-// LDS written and read by one wave alone: its accesses happen in order, the
-// compiler is told to keep them so.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <int W, long FLAG>
 __global__ __launch_bounds__(kWave* kSymFarWaves, 2) void sakura_far_sym_kernel(SakuraArgs a)
 {

@@ -488,6 +488,15 @@ __device__ __forceinline__ void wave_ror1(double (&v)[K])
     }
 }
 
+// LDS written and read by one wave alone: its accesses happen in order, the
+// compiler is told to keep them so.
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <class S>
 __device__ __forceinline__ double sym_join(double t, double v, int k)
 {
@@ -525,6 +534,8 @@ __device__ __forceinline__ void sym_pass(const typename S::T* slot, int lane,
             }
         }
         const int j = (lane - (s0 + kRun - 1)) & (kWave - 1);
+        // j's sum of the runs before was written by another lane
+        if (s0 > 0) wave_lds_sync();
 #pragma unroll
         for (int k = 0; k < S::kK; ++k) {
             const double v = static_cast<double>(aj[k]) * S::scale();
