@@ -44,12 +44,26 @@ constexpr int kSymWaves = kSymBlock / kWave;
 // aj, e2u, eta) adding the pair to both particles' sums.  kU: the pair
 // softening is e2u; kM: pairs at zero separation are masked.
 
+// A padding particle is a copy of the set's last one without mass, softened
+// enough that no pair with it overflows (infinity times its zero mass would
+// be NaN in the real particle's sum).  A uniform tile has the set's softening
+// for it too, where that is enough (pad_ok; an unmasked tile runs only where
+// every pair is finite); else the tile takes the general loop.  kPadSafe: a
+// policy whose padding needs none of this (1/R of a potential does not
+// overflow; a padding particle without position has no time step).
+template <int kM0, int kE2, class T, int F>
+__device__ __forceinline__ void sym_pad(T (&f)[F])
+{
+    f[kM0] = T(0);
+    f[kE2] = T(1);
+}
+
 template <class P>
 struct SymPhi {
     using Base = OpPhi<P>;
     using T = typename P::T;
     static constexpr int kF = 5, kK = 1, kE2 = 4, kM0 = 0;
-    static constexpr bool kMax1 = false;
+    static constexpr bool kMax1 = false, kPadSafe = true;
     __device__ static void load(const typename Base::Args& a, const typename Base::Frame&, int i,
                                 T (&f)[kF])
     {
@@ -77,14 +91,14 @@ struct SymAcc {
     using Base = OpAcc<P>;
     using T = typename P::T;
     static constexpr int kF = 5, kK = 3, kE2 = 4, kM0 = 0;
-    static constexpr bool kMax1 = false;
+    static constexpr bool kMax1 = false, kPadSafe = false;
     __device__ static void load(const typename Base::Args& a, const typename Base::Frame&, int i,
                                 T (&f)[kF])
     {
 #pragma unroll
         for (int k = 0; k < kF; ++k) f[k] = a.ip[k][i];
     }
-    __device__ static void pad(T (&f)[kF]) { f[0] = T(0); }
+    __device__ static void pad(T (&f)[kF]) { sym_pad<kM0, kE2>(f); }
     template <bool kU, bool kM>
     __device__ static __forceinline__ void interact(const T (&I)[kF], const T (&J)[kF],
                                                     T (&ai)[kK], T (&aj)[kK], T e2u, T)
@@ -111,14 +125,14 @@ struct SymAccJerk {
     using Base = OpAccJerk<P>;
     using T = typename P::T;
     static constexpr int kF = 8, kK = 6, kE2 = 4, kM0 = 0;
-    static constexpr bool kMax1 = false;
+    static constexpr bool kMax1 = false, kPadSafe = false;
     __device__ static void load(const typename Base::Args& a, const typename Base::Frame&, int i,
                                 T (&f)[kF])
     {
 #pragma unroll
         for (int k = 0; k < kF; ++k) f[k] = a.ip[k][i];
     }
-    __device__ static void pad(T (&f)[kF]) { f[0] = T(0); }
+    __device__ static void pad(T (&f)[kF]) { sym_pad<kM0, kE2>(f); }
     template <bool kU, bool kM>
     __device__ static __forceinline__ void interact(const T (&I)[kF], const T (&J)[kF],
                                                     T (&ai)[kK], T (&aj)[kK], T e2u, T)
@@ -157,14 +171,14 @@ struct SymSnapCrackle {
     using Base = OpSnapCrackle<P>;
     using T = typename P::T;
     static constexpr int kF = 14, kK = 6, kE2 = 4, kM0 = 0;
-    static constexpr bool kMax1 = false;
+    static constexpr bool kMax1 = false, kPadSafe = false;
     __device__ static void load(const typename Base::Args& a, const typename Base::Frame&, int i,
                                 T (&f)[kF])
     {
 #pragma unroll
         for (int k = 0; k < kF; ++k) f[k] = a.ip[k][i];
     }
-    __device__ static void pad(T (&f)[kF]) { f[0] = T(0); }
+    __device__ static void pad(T (&f)[kF]) { sym_pad<kM0, kE2>(f); }
     template <bool kU, bool kM>
     __device__ static __forceinline__ void interact(const T (&I)[kF], const T (&J)[kF],
                                                     T (&ai)[kK], T (&aj)[kK], T e2u, T)
@@ -198,7 +212,7 @@ struct SymTstep {
     using Base = OpTstep<P>;
     using T = typename P::T;
     static constexpr int kF = 8, kK = 2, kE2 = 4, kM0 = 0;
-    static constexpr bool kMax1 = true;
+    static constexpr bool kMax1 = true, kPadSafe = true;
     __device__ static void load(const typename Base::Args& a, const typename Base::Frame&, int i,
                                 T (&f)[kF])
     {
@@ -241,12 +255,12 @@ struct SymSplitAcc {
     using Base = OpSplitAcc;
     using T = float;
     static constexpr int kF = 8, kK = 3, kE2 = 7, kM0 = 3;
-    static constexpr bool kMax1 = false;
+    static constexpr bool kMax1 = false, kPadSafe = false;
     __device__ static void load(const Base::Args& a, const Base::Frame& fr, int i, T (&f)[kF])
     {
         split_fields<Base>(a, fr, i, f);
     }
-    __device__ static void pad(T (&f)[kF]) { f[3] = 0.0f; }
+    __device__ static void pad(T (&f)[kF]) { sym_pad<kM0, kE2>(f); }
     template <bool kU, bool kM>
     __device__ static __forceinline__ void interact(const T (&I)[kF], const T (&J)[kF],
                                                     T (&ai)[kK], T (&aj)[kK], T e2u, T)
@@ -271,12 +285,12 @@ struct SymSplitAccJerk {
     using Base = OpSplitAccJerk;
     using T = float;
     static constexpr int kF = 11, kK = 6, kE2 = 7, kM0 = 3;
-    static constexpr bool kMax1 = false;
+    static constexpr bool kMax1 = false, kPadSafe = false;
     __device__ static void load(const Base::Args& a, const Base::Frame& fr, int i, T (&f)[kF])
     {
         split_fields<Base>(a, fr, i, f);
     }
-    __device__ static void pad(T (&f)[kF]) { f[3] = 0.0f; }
+    __device__ static void pad(T (&f)[kF]) { sym_pad<kM0, kE2>(f); }
     template <bool kU, bool kM>
     __device__ static __forceinline__ void interact(const T (&I)[kF], const T (&J)[kF],
                                                     T (&ai)[kK], T (&aj)[kK], T e2u, T)
@@ -313,7 +327,7 @@ struct SymSplitTstep {
     using Base = OpSplitTstep;
     using T = float;
     static constexpr int kF = 11, kK = 2, kE2 = 7, kM0 = 3;
-    static constexpr bool kMax1 = true;
+    static constexpr bool kMax1 = true, kPadSafe = true;
     // masses held doubled, as OpSplitTstep's
     __device__ static void load(const Base::Args& a, const Base::Frame& fr, int i, T (&f)[kF])
     {
@@ -568,10 +582,12 @@ __device__ __forceinline__ void sym_body(const typename S::Base::Args& a, int bi
     T I[W][S::kF];
     T ai[W][S::kK];
     double di[W][S::kK];
+    [[maybe_unused]] T e2_i[W];
 #pragma unroll
     for (int w = 0; w < W; ++w) {
         const int i = ibase + w * kSymBlock + tid;
         S::load(a, fr, i < n ? i : n - 1, I[w]);
+        e2_i[w] = I[w][S::kE2];
         if (i >= n) S::pad(I[w]);
 #pragma unroll
         for (int k = 0; k < S::kK; ++k) {
@@ -589,10 +605,16 @@ __device__ __forceinline__ void sym_body(const typename S::Base::Args& a, int bi
     T e2_first = T(0);
     [[maybe_unused]] bool unmask = false;
     [[maybe_unused]] T y_self = T(0);
+    [[maybe_unused]] bool pad_ok = true;  // no uniform tile overflows at a padding particle
     if constexpr (kUni) {
         e2_first = Op::e2_of_i(a, ibase);
+        if constexpr (!kUnmask && !S::kPadSafe) {
+            const T y = rsqrt_refined(e2_first + e2_first);
+            pad_ok = __builtin_isfinite(y * y * y);
+        }
 #pragma unroll
-        for (int w = 0; w < W; ++w) iuni = iuni && I[w][S::kE2] == e2_first;
+        for (int w = 0; w < W; ++w) iuni = iuni && e2_i[w] == e2_first;
+        iuni = iuni && (pad_ok || ibase + BI <= n);
     }
     if constexpr (kUnmask) unmask = Op::unmask_allowed(a);
     if constexpr (kSelf) {
@@ -606,6 +628,9 @@ __device__ __forceinline__ void sym_body(const typename S::Base::Args& a, int bi
     const int t0 = static_cast<int>(static_cast<long long>(row_tiles) * chunk / a.nsplit);
     const int t1 = static_cast<int>(static_cast<long long>(row_tiles) * (chunk + 1) / a.nsplit);
     double* jpart = a.partial + static_cast<size_t>(a.nsplit) * S::kK * n;
+    // vmcnt(0): the i-particles' loads end here, or the compiler waits for
+    // them in the pair loop, on every pass through it (float Phi: 2 %)
+    __builtin_amdgcn_s_waitcnt(0x0f70);
     for (int t = t0; t < t1; ++t) {
         const int d = t / (BI / TJ);
         int jblock = row + d;
@@ -619,8 +644,8 @@ __device__ __forceinline__ void sym_body(const typename S::Base::Args& a, int bi
             T f[S::kF];
             const int j = j0 + tid;
             S::load(a, fr, j < n ? j : n - 1, f);
-            if (j >= n) S::pad(f);
             if constexpr (kUni) tuni = tuni && f[S::kE2] == e2_first;
+            if (j >= n) S::pad(f);
             if constexpr (kSelf) tsafe = tsafe && Op::self_safe_m(y_self, f[S::kM0]);
             T* dst = slots + (tid / kWave) * kSubLen + lane;
 #pragma unroll
@@ -633,7 +658,7 @@ __device__ __forceinline__ void sym_body(const typename S::Base::Args& a, int bi
         if constexpr (kUnmask) {
             special = __syncthreads_and(tuni && tsafe);
         } else if constexpr (kUni) {
-            special = __syncthreads_and(tuni);
+            special = __syncthreads_and(tuni) && (pad_ok || j0 + TJ <= n);
         } else {
             __syncthreads();
         }
