@@ -403,7 +403,14 @@ static int launch_tuned(const Launcher<Op> (&table)[kShapes], int kernel, int sl
     const int* d = shape_dims(kernel, g_tune[kernel][slot][b].shape);
     if (pads_rows(a.ni, d[0], d[1])) b = 0;
     const TuneEntry& t = g_tune[kernel][slot][b];
-    return table[t.shape](a, s, bucket_wg(b, a.ni, t.wg_per_cu), fixed);
+    int wg = bucket_wg(b, a.ni, t.wg_per_cu);
+    // a seed's initial conditions keep their bits (sym.h: kSymOpAbove): FP64
+    // Phi of a set against itself below 2^22 pairs in the four workgroups per
+    // CU its splits had
+    if constexpr (std::is_same<Op, OpPhi<Fast64>>::value) {
+        if (wg > 4 && a.ni < 2048 && same_set(a)) wg = 4;
+    }
+    return table[t.shape](a, s, wg, fixed);
 }
 
 #define TUPAN_RUN(Op, SHAPES, kernel, slot)                                      \

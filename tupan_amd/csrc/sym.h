@@ -377,8 +377,8 @@ constexpr bool kHasSym = !std::is_void<typename SymOf<Op>::type>::value;
 // Largest set an op leaves to the tile engine whatever the plan below says.
 // Initial conditions are drawn from the FP64 Phi, and the 1e-14 comparison of
 // two pair solvers on the 16384-particle realisation depends on its last
-// bits, so a seed's realisation keeps the tile engine's summation order up to
-// 2^15 particles, where a potential costs under 0.7 ms (n = 32768: 0.67 there,
+// bits, so a seed's realisation keeps the tile engine's summation order (and
+// its j-splits: pairwise.hip, launch_tuned) up to 2^15 particles, where a potential costs under 0.7 ms (n = 32768: 0.67 there,
 // 0.40 here); beyond, the time counts (n = 50000: 1.49 against 0.87 ms).
 template <class Op>
 inline constexpr int kSymOpAbove = 0;
