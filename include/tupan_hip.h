@@ -24,7 +24,10 @@
  *
  * Output arrays are overwritten, never accumulated into.  Kernels keep no
  * pointer past the call.  The device layer uses a per-device scratch
- * workspace for j-split partial sums (and, for Acc-Jerk calls of at least
+ * workspace for partial sums: j-splits, the sums of a set against itself (up
+ * to 4 GiB above a few hundred thousand particles; a call whose sums would
+ * take more, or for which the workspace cannot grow, splits j instead) and
+ * the Sakura pair drift's entries and near-pair lists (up to 9 GiB) (and, for Acc-Jerk calls of at least
  * 2^28 pairs in the fp64 and split32 modes, the hash table of a scan for
  * particles that share a position: it decides whether the pair loop may
  * leave out the test that drops zero-separation pairs; the sums are the

@@ -52,10 +52,10 @@ __device__ __forceinline__ double sakura_dt(const SakuraArgs& a)
 // pairs that are not listed, from the plain guess and unlogged: with a guess
 // network or a log all but the first kNearSlots, else all of them (a wave
 // that solves the whole entry has more of its lanes busy, and spares the
-// list: N = 9000, every pair near: 9.6 ms with the first 32 of each entry
-// listed, 5.2 ms whole).  Fewer slots make entries of ordinary states
+// list: N = 9000, every pair near: 9.5 ms with the first 32 of each entry
+// listed, 5.0 ms whole).  Fewer slots make entries of ordinary states
 // over-full, of whose candidates few are near (N = 6000 with a fifth of the
-// particles slow: 402 us with 32 slots, 735 with 8, 450 in the tile form).
+// particles slow: 364 us with 32 slots, 735 with 8, 450 in the tile form).
 constexpr int kNearSlots = 32;
 
 __device__ __forceinline__ int near_listed(int count, int whole)

@@ -183,8 +183,8 @@ struct SymSnapCrackle {
     __device__ static __forceinline__ void interact(const T (&I)[kF], const T (&J)[kF],
                                                     T (&ai)[kK], T (&aj)[kK], T e2u, T)
     {
-        // both particles' terms are w times the same six values: the op's
-        // own pair with unit mass, from zero sums, gives minus them
+        // both particles' terms are the same six values times 1/R^3 and the
+        // other's mass
         typename Base::IReg r;
         typename Base::Slot s;
         typename Base::Acc c;
@@ -378,8 +378,9 @@ constexpr bool kHasSym = !std::is_void<typename SymOf<Op>::type>::value;
 // Initial conditions are drawn from the FP64 Phi, and the 1e-14 comparison of
 // two pair solvers on the 16384-particle realisation depends on its last
 // bits, so a seed's realisation keeps the tile engine's summation order (and
-// its j-splits: pairwise.hip, launch_tuned) up to 2^15 particles, where a potential costs under 0.7 ms (n = 32768: 0.67 there,
-// 0.40 here); beyond, the time counts (n = 50000: 1.49 against 0.87 ms).
+// its j-splits: pairwise.hip, launch_tuned) up to 2^15 particles, where a
+// potential costs under 0.7 ms (n = 32768: 0.67 there, 0.40 here); beyond,
+// the time counts (n = 50000: 1.49 against 0.87 ms).
 template <class Op>
 inline constexpr int kSymOpAbove = 0;
 template <>
@@ -418,7 +419,10 @@ __host__ __device__ inline size_t sym_doubles(const SymPlan& p, int nk, int n)
 // and 94 us at 9500, 824 and 873 us (W = 2, 4) at 32001, 1339 and 1285 us at
 // 41000; the FP32 forms fill the ALU best with the four waves per SIMD that
 // W = 2 leaves room for, and take W = 4 only where it halves a partial-sum
-// array of several hundred MB at equal speed.
+// array of several hundred MB at equal speed.  One rule serves every op of an
+// arithmetic; off it by most is FP64 SnapCrackle, whose W = 4 holds one wave
+// per SIMD: 2.97 ms at n = 37000, 2.58 under W = 2 (9.0 and 8.3 at 70000; tile
+// engine 3.9 and 14.0).
 // The bounds are multiples of the smaller shape's block, so every block
 // count of a shape occurs at a whole multiple of its block.
 constexpr int kSymAbove64 = 2048, kSymAbove32 = 4096;

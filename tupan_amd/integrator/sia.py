@@ -48,7 +48,7 @@ import logging
 import torch
 
 from . import Base
-from .device_update import device_update, on_current_device
+from .device_update import BOOK, DRIFT, device_update, on_current_device
 from .fewbody import FewBody
 
 SUBTREE_MAX = 64
@@ -174,8 +174,8 @@ def join(slow, fast):
 
 def drift(ips, tau):
     """sia.py:162-171 with drift_n and drift_pn (sia.py:64-101)."""
-    if not device_update(0, (ips.rx, ips.ry, ips.rz, ips.vx, ips.vy, ips.vz),
-                          tau):
+    if not device_update(DRIFT, (ips.rx, ips.ry, ips.rz,
+                                 ips.vx, ips.vy, ips.vz), tau):
         ips.rx += ips.vx * tau
         ips.ry += ips.vy * tau
         ips.rz += ips.vz * tau
@@ -185,8 +185,8 @@ def drift(ips, tau):
 
 
 def kick_n(ips, tau):
-    if not device_update(0, (ips.vx, ips.vy, ips.vz, ips.ax, ips.ay, ips.az),
-                          tau):
+    if not device_update(DRIFT, (ips.vx, ips.vy, ips.vz,
+                                 ips.ax, ips.ay, ips.az), tau):
         ips.vx += ips.ax * tau
         ips.vy += ips.ay * tau
         ips.vz += ips.az * tau
@@ -454,7 +454,8 @@ class SIA(Base):
             else:
                 type(ps).t_curr += tau
         if slow.n:
-            if not device_update(1, (slow.tstep, slow.time, slow.nstep), tau):
+            if not device_update(BOOK, (slow.tstep, slow.time, slow.nstep),
+                                 tau):
                 slow.tstep[...] = tau
                 slow.time += tau
                 slow.nstep += 1
@@ -801,7 +802,9 @@ class _DeviceSubtree(object):
 
     def begin(self, ps):
         """The step's start: the time, and cleared counters and status.  The
-        time is advanced on the device until end()."""
+        time is advanced on the device until end(); a step that fails (a
+        subtree's status is read with the next partition's count and at the
+        step's end) leaves the class's t_curr where the step began."""
         names = list(ps.arrays())
         self.roles = (ctypes.c_int * len(SUBTREE_ROLES))(
             *[names.index(r) for r in SUBTREE_ROLES])
