@@ -13,17 +13,17 @@ def device_update(kind, tensors, h=0.0):
     """One update of ``tensors`` (tupan_sia_update's arrays, in its order):
     DRIFT x += v h, BOOK, HALF_DRIFT x += (v h) / 2, ADD x += d.  The values
     are the array operations', bit for bit.  False, and nothing done, unless
-    they are contiguous 8-byte arrays of one size on the current device: the
-    caller then runs the same operations array by array."""
+    they are contiguous float64 arrays (BOOK's third: int64) of one size on
+    the current device: the caller then runs the same operations array by
+    array."""
     if not on_current_device(tensors[0]):
         return False
     n = tensors[0].numel()
-    for t in tensors:
-        if not (t.is_cuda and t.element_size() == 8 and t.is_contiguous()
+    for k, t in enumerate(tensors):
+        dtype = torch.int64 if kind == BOOK and k == 2 else torch.float64
+        if not (t.is_cuda and t.dtype == dtype and t.is_contiguous()
                 and t.numel() == n and not t.requires_grad):
             return False
-    if kind != BOOK and any(t.dtype != torch.float64 for t in tensors):
-        return False
     from .. import _native
     from ..lib.hip_backend import current_stream_handle
     _native.check(_native.lib().tupan_sia_update(

@@ -780,6 +780,11 @@ class _DeviceSubtree(object):
             return None
         if any(r not in arrays for r in SUBTREE_ROLES) or len(arrays) > 32:
             return None
+        # nstep is the one integer among the roles
+        if any(arrays[r].dtype != (torch.int64 if r == "nstep"
+                                   else torch.float64)
+               for r in SUBTREE_ROLES):
+            return None
         return cls(sia, kernels[0].mode, kernels[1].mode, ps.device)
 
     def __init__(self, sia, acc_mode, tstep_mode, device):
